@@ -31,6 +31,9 @@ RC, RL, MARGIN = 9.0, 8.0, 0.5
 MODELS = ("TIP3P", "TIP4P", "TIP5P")
 PERIODIC = {0: (True, True, True), 1: (False, False, True), 2: (True, True, False)}
 SGM_WALL, EPS_WALL, RHO_WALL, NFWALL = 3.277, 0.3886, 0.38016, 1000
+# pressure ladder (Pa); the TIP5P of inputs.MOLTYPE binds weakly and boils
+# under the barostat at ordinary pressures
+PRESSURE = {"TIP3P": (0.1e6, 150e6), "TIP4P": (0.1e6, 150e6), "TIP5P": (400e6, 800e6)}
 # FLOP of one ordered molecule pair inside the cutoff, FMA = 2 (one LJ site
 # term 32, each Coulomb site term 27, 38 per pair)
 PAIR_FLOPS = {"TIP3P": 313, "TIP4P": 313, "TIP5P": 502}
@@ -66,13 +69,13 @@ def listed():
         dict(name="slit512-tip5p-fp64", kind="interval", precision=1, intervals=1, steps=100,
              **_job(2, "TIP5P", 512, 32, 4, 10.0, 40.0)),
         # large replicas of the served stream: a bulk and a slit job whose
-        # states exceed one workgroup's LDS, and its largest model and size
+        # states exceed one workgroup's LDS, and a bulk job of its largest size
         dict(name="bulk1820-tip4p-16rep", kind="interval", precision=0, intervals=1, steps=100,
              **_job(0, "TIP4P", 1820, 16, 1)),
         dict(name="slit1374-tip5p-64rep", kind="interval", precision=0, intervals=1, steps=100,
              **_job(2, "TIP5P", 1374, 64, 1, 14.0)),
-        dict(name="bulk2048-tip5p-8rep", kind="interval", precision=0, intervals=1, steps=100,
-             **_job(0, "TIP5P", 2048, 8, 1)),
+        dict(name="bulk2048-tip4p-8rep", kind="interval", precision=0, intervals=1, steps=100,
+             **_job(0, "TIP4P", 2048, 8, 1)),
         # eight unequal tubes of two models, 32 replicas each, in one batch
         dict(name="uneven-tubes-256rep", kind="batch", precision=0, intervals=2, steps=100, first=5, jobs=8, ntemp=8,
              npress=4),
@@ -126,7 +129,7 @@ def _geometry(job):
         Lxy = 2.0 * (size + 9.0) + 4.0
         return (Lxy, Lxy, Lz), size - 2.8
     Lxy = length or max(math.sqrt(n * 29.9 / (size - 3.4)), 2 * (RC + MARGIN) + 1.0)
-    return (Lxy, Lxy, size + 40.0), 0.5 * (size - 3.4)
+    return (Lxy, Lxy, size + 40.0), 0.5 * size - 2.6
 
 
 def _lattice(job, rng):
@@ -175,7 +178,7 @@ def _rotate(q, b):
     return (m.unsqueeze(-3) * b.view(*([1] * (q.dim() - 1)), -1, 1, 3)).sum(-1), m
 
 
-def _relaxed(job, rng, steps=120):
+def _relaxed(job, rng, steps=200):
     """Rigid-body descent of one configuration: every molecule moves down the
     gradient of its energy with its 40 nearest neighbours held fixed."""
     x0, box, acc = _lattice(job, rng)
@@ -222,7 +225,7 @@ def _system(job, seed, steps=100):
     rng = np.random.RandomState(seed % (1 << 31))
     x, q, box, mt = _relaxed(job, rng)
     T, P = inputs.make_ladder(job["ntemp"], job["npress"], inputs.geometric(240.0, 340.0, job["ntemp"]),
-                              inputs.geometric(0.1e6, 150e6, job["npress"]))
+                              inputs.geometric(*PRESSURE[job["model"]], job["npress"]))
     conf = job["confined"]
     s = inputs.System(job["model"], job["nmol"], 1, (1, 2, 3)[conf] if job["barostat"] else 0, conf, 2.0, RC, RL, steps,
                       job["ntemp"], job["npress"], T, P)
