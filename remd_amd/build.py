@@ -16,7 +16,9 @@ CSRC = os.path.join(PKG, "csrc")
 LIB = os.path.join(PKG, "libremd_gpu.so")
 DRIVER = os.path.join(PKG, "remd_md")
 
-HIP_SOURCES = ["remd_kernels.hip", "remd_engine.hip"]
+# (source, object, defines): the kernels compile in units, side by side
+HIP_UNITS = [("remd_kernels.hip", f"remd_kernels_{k}.o", [f"-DREMD_UNIT={k}"]) for k in (5, 3, 4, 2, 1)]
+HIP_UNITS.append(("remd_engine.hip", "remd_engine.o", []))
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("REMD_OFFLOAD_ARCH", "gfx950")
 
@@ -43,18 +45,19 @@ def _run(cmd, cwd=None):
 
 
 def build_library(verbose=False):
-    """Compile each HIP source to an object (in parallel), then link."""
+    """Compile each unit to an object (in parallel), then link."""
     from concurrent.futures import ThreadPoolExecutor
 
     objdir = os.path.join(PKG, "_build")
     os.makedirs(objdir, exist_ok=True)
 
-    def compile_one(s):
-        obj = os.path.join(objdir, os.path.splitext(s)[0] + ".o")
-        return obj, _run([HIPCC, *HIP_FLAGS, "-c", "-o", obj, os.path.join(CSRC, s)])
+    def compile_one(u):
+        src, name, defines = u
+        obj = os.path.join(objdir, name)
+        return obj, _run([HIPCC, *HIP_FLAGS, *defines, "-c", "-o", obj, os.path.join(CSRC, src)])
 
-    with ThreadPoolExecutor(len(HIP_SOURCES)) as ex:
-        done = list(ex.map(compile_one, HIP_SOURCES))
+    with ThreadPoolExecutor(len(HIP_UNITS)) as ex:
+        done = list(ex.map(compile_one, HIP_UNITS))
     tmp = LIB + ".tmp"
     out = _run([HIPCC, *HIP_FLAGS, "-shared", "-o", tmp, *[o for o, _ in done]])
     os.replace(tmp, LIB)

@@ -24,7 +24,24 @@
 
 #include "remd_common.h"
 
+// The file is compiled once per unit (REMD_UNIT), so that its kernel
+// instantiations build in parallel.
+#define REMD_UNIT_MISC 1
+#define REMD_UNIT_INTERVAL 2
+#define REMD_UNIT_RESIDENT_FIXED 3
+#define REMD_UNIT_RESIDENT 4
+#define REMD_UNIT_BATCH 5
+#ifndef REMD_UNIT
+#error "REMD_UNIT selects the kernels of this compilation"
+#endif
+
 namespace remd {
+
+// host addresses of the kernels of the other units
+const void *interval_fn(int nt, int nsite, int prec);
+const void *resident_fn_fixed(int nsite, int ens);
+const void *resident_fn_runtime(int nsite, int prec);
+const void *resident_batch_fn();
 
 constexpr int WAVE = 64;
 
@@ -2359,6 +2376,7 @@ __device__ inline bool run_resident_fixed(unsigned variant, const LaunchArgs &a,
   }
 }
 
+#if REMD_UNIT == REMD_UNIT_BATCH
 __global__ __launch_bounds__(RNT) void resident_batch_kernel(LaunchArgs a) {
   extern __shared__ __align__(16) char smem[];
   const unsigned e = a.blk[blockIdx.x];
@@ -2399,6 +2417,10 @@ __global__ __launch_bounds__(RNT) void resident_batch_kernel(LaunchArgs a) {
   }
 }
 
+const void *resident_batch_fn() { return (const void *)resident_batch_kernel; }
+#endif  // REMD_UNIT_BATCH
+
+#if REMD_UNIT == REMD_UNIT_MISC
 // ---------------------------------------------------------------- b1
 // ForceCalculator::CalcWallForce, tube (src/force_calculator.cxx:117-161):
 // one thread per table node, 10000-point phi sum in FP64 with float sqrt as
@@ -2615,41 +2637,51 @@ __global__ void scratch_setup_kernel(const ReplicaDesc *src, ReplicaDesc *dst, i
     blk[k] = rep < nrep ? ((unsigned)rep << 12 | variant << 8 | (unsigned)parts << 4 | (unsigned)part) : ~0u;
   }
 }
+#endif  // REMD_UNIT_MISC
 
-// ------------------------------------------------------------ launchers
+// -------------------------------------------------------- kernel addresses
+#if REMD_UNIT == REMD_UNIT_INTERVAL
 // Kernel class of a replica: (block threads, sites, pair precision).
 template <int NT>
-static hipError_t launch_nt(const LaunchArgs &a, int nsite, int prec, int lds, hipStream_t st) {
-  const dim3 g(a.nrep), b(NT);
-  const int key = nsite * 2 + prec;
-  switch (key) {
-    case 6: hipLaunchKernelGGL((interval_kernel<NT, 3, float>), g, b, lds, st, a); break;
-    case 8: hipLaunchKernelGGL((interval_kernel<NT, 4, float>), g, b, lds, st, a); break;
-    case 10: hipLaunchKernelGGL((interval_kernel<NT, 5, float>), g, b, lds, st, a); break;
-    case 7: hipLaunchKernelGGL((interval_kernel<NT, 3, double>), g, b, lds, st, a); break;
-    case 9: hipLaunchKernelGGL((interval_kernel<NT, 4, double>), g, b, lds, st, a); break;
-    case 11: hipLaunchKernelGGL((interval_kernel<NT, 5, double>), g, b, lds, st, a); break;
-    default: return hipErrorInvalidValue;
+static const void *interval_fn_nt(int nsite, int prec) {
+  switch (nsite * 2 + prec) {
+    case 6: return (const void *)interval_kernel<NT, 3, float>;
+    case 8: return (const void *)interval_kernel<NT, 4, float>;
+    case 10: return (const void *)interval_kernel<NT, 5, float>;
+    case 7: return (const void *)interval_kernel<NT, 3, double>;
+    case 9: return (const void *)interval_kernel<NT, 4, double>;
+    case 11: return (const void *)interval_kernel<NT, 5, double>;
+    default: return nullptr;
   }
-  return hipGetLastError();
 }
 
-// Resident path: block size 256 only.  The FP32 jobs of the ensembles
-// ENS_*_NP run an instantiation with the modes fixed, the rest the one that
-// reads them from the job (same bits either way).
-static const void *resident_fn(int nsite, int prec, int ens) {
-  if (prec == 0) {
+const void *interval_fn(int nt, int nsite, int prec) {
+  if (nt == 256) return interval_fn_nt<256>(nsite, prec);
+  if (nt == 512) return interval_fn_nt<512>(nsite, prec);
+  if (nt == 128) return interval_fn_nt<128>(nsite, prec);
+  return nullptr;
+}
+#endif
+
+#if REMD_UNIT == REMD_UNIT_RESIDENT_FIXED
+// FP32 jobs of the ensembles ENS_*_NP: the modes are fixed.
+const void *resident_fn_fixed(int nsite, int ens) {
 #define REMD_RES_ENS(E)                                                  \
   if (ens == E) {                                                        \
     if (nsite == 3) return (const void *)resident_kernel<RNT, 3, float, E>; \
     if (nsite == 4) return (const void *)resident_kernel<RNT, 4, float, E>; \
     if (nsite == 5) return (const void *)resident_kernel<RNT, 5, float, E>; \
   }
-    REMD_RES_ENS(ENS_TUBE_NP)
-    REMD_RES_ENS(ENS_SLIT_NP)
-    REMD_RES_ENS(ENS_BULK_NP)
+  REMD_RES_ENS(ENS_TUBE_NP)
+  REMD_RES_ENS(ENS_SLIT_NP)
+  REMD_RES_ENS(ENS_BULK_NP)
 #undef REMD_RES_ENS
-  }
+  return nullptr;
+}
+#endif
+
+#if REMD_UNIT == REMD_UNIT_RESIDENT
+const void *resident_fn_runtime(int nsite, int prec) {
   switch (nsite * 2 + prec) {
     case 6: return (const void *)resident_kernel<RNT, 3, float>;
     case 8: return (const void *)resident_kernel<RNT, 4, float>;
@@ -2660,6 +2692,25 @@ static const void *resident_fn(int nsite, int prec, int ens) {
     default: return nullptr;
   }
 }
+#endif
+
+#if REMD_UNIT == REMD_UNIT_MISC
+// ------------------------------------------------------------ launchers
+// Resident path: block size 256 only.  The FP32 jobs of the ensembles
+// ENS_*_NP run an instantiation with the modes fixed, the rest the one that
+// reads them from the job (same bits either way).
+static const void *resident_fn(int nsite, int prec, int ens) {
+  const void *f = prec == 0 ? resident_fn_fixed(nsite, ens) : nullptr;
+  return f ? f : resident_fn_runtime(nsite, prec);
+}
+
+static hipError_t launch_fn(const void *f, int grid, int nt, const LaunchArgs &a, int lds, hipStream_t st) {
+  if (!f) return hipErrorInvalidValue;
+  LaunchArgs arg = a;
+  void *args[] = {&arg};
+  const hipError_t e = hipLaunchKernel(f, dim3(grid), dim3(nt), args, (size_t)lds, st);
+  return e != hipSuccess ? e : hipGetLastError();
+}
 
 int resident_grid(int nrep, int parts) { return parts <= 1 ? nrep : 8 * parts * ((nrep + 7) / 8); }
 
@@ -2669,22 +2720,16 @@ int resident_lds(int nmol, int nsite, int prec, int site_dbg, int gm) {
 
 hipError_t launch_resident(const LaunchArgs &a, int nsite, int prec, int ens, int lds, hipStream_t st) {
   if (a.nrep <= 0) return hipSuccess;
-  const void *f = resident_fn(nsite, prec, ens);
-  if (!f) return hipErrorInvalidValue;
-  LaunchArgs arg = a;
-  void *args[] = {&arg};
-  const hipError_t e = hipLaunchKernel(f, dim3(resident_grid(a.nrep, a.parts)), dim3(RNT), args, (size_t)lds, st);
-  return e != hipSuccess ? e : hipGetLastError();
+  return launch_fn(resident_fn(nsite, prec, ens), resident_grid(a.nrep, a.parts), RNT, a, lds, st);
 }
 
 hipError_t launch_resident_batch(const LaunchArgs &a, int lds, hipStream_t st) {
   if (a.nblk <= 0 || !a.blk) return hipSuccess;
-  hipLaunchKernelGGL(resident_batch_kernel, dim3(a.nblk), dim3(RNT), lds, st, a);
-  return hipGetLastError();
+  return launch_fn(resident_batch_fn(), a.nblk, RNT, a, lds, st);
 }
 
 hipError_t resident_batch_occupancy(int lds, int *per_cu) {
-  return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, (const void *)resident_batch_kernel, RNT,
+  return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, resident_batch_fn(), RNT,
                                                       (size_t)lds);
 }
 
@@ -2697,27 +2742,7 @@ hipError_t resident_occupancy(int nsite, int prec, int ens, int lds, int *per_cu
 
 hipError_t launch_interval(const LaunchArgs &a, int nt, int nsite, int prec, int lds, hipStream_t st) {
   if (a.nrep <= 0) return hipSuccess;
-  if (nt == 256) return launch_nt<256>(a, nsite, prec, lds, st);
-  if (nt == 512) return launch_nt<512>(a, nsite, prec, lds, st);
-  if (nt == 128) return launch_nt<128>(a, nsite, prec, lds, st);
-  return hipErrorInvalidValue;
-}
-
-template <int NT>
-static hipError_t set_lds_nt(int bytes) {
-  hipError_t e = hipSuccess;
-#define REMD_SETLDS(NS_, PT_)                                                                              \
-  if (e == hipSuccess)                                                                                      \
-    e = hipFuncSetAttribute((const void *)interval_kernel<NT, NS_, PT_>,                                    \
-                            hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-  REMD_SETLDS(3, float)
-  REMD_SETLDS(4, float)
-  REMD_SETLDS(5, float)
-  REMD_SETLDS(3, double)
-  REMD_SETLDS(4, double)
-  REMD_SETLDS(5, double)
-#undef REMD_SETLDS
-  return e;
+  return launch_fn(interval_fn(nt, nsite, prec), a.nrep, nt, a, lds, st);
 }
 
 hipError_t set_kernel_lds_limit(int bytes) {
@@ -2728,11 +2753,12 @@ hipError_t set_kernel_lds_limit(int bytes) {
       for (int pr = 0; pr < 2 && e == hipSuccess; pr++)
         e = hipFuncSetAttribute(resident_fn(ns, pr, ens[k]), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
   if (e == hipSuccess)
-    e = hipFuncSetAttribute((const void *)resident_batch_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+    e = hipFuncSetAttribute(resident_batch_fn(), hipFuncAttributeMaxDynamicSharedMemorySize,
                             bytes);
-  if (e == hipSuccess) e = set_lds_nt<256>(bytes);
-  if (e == hipSuccess) e = set_lds_nt<512>(bytes);
-  if (e == hipSuccess) e = set_lds_nt<128>(bytes);
+  for (int nt = 128; nt <= 512 && e == hipSuccess; nt *= 2)
+    for (int ns = 3; ns <= 5 && e == hipSuccess; ns++)
+      for (int pr = 0; pr < 2 && e == hipSuccess; pr++)
+        e = hipFuncSetAttribute(interval_fn(nt, ns, pr), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
   if (e == hipSuccess)
     e = hipFuncSetAttribute((const void *)sort_window_kernel<256>, hipFuncAttributeMaxDynamicSharedMemorySize,
                             bytes);
@@ -2778,5 +2804,7 @@ hipError_t launch_exchange(const ExchangeJob *jobs, int njobs, hipStream_t st) {
   hipLaunchKernelGGL(exchange_kernel, dim3(njobs), dim3(256), 0, st, jobs, njobs);
   return hipGetLastError();
 }
+
+#endif  // REMD_UNIT_MISC
 
 }  // namespace remd
