@@ -107,22 +107,26 @@ constexpr int RNT = 256;
 // the radix sort rather than the rank sort.
 constexpr int RADIX_MIN_DEFAULT = 768;
 
-// Ensemble code of a job: tconstant 0..2, pconstant 0..3, confined 0..2;
-// ENS_RUNTIME: the modes are read from the job.
+// Ensemble code of a job: tconstant 0..2, pconstant 0..3, confined 0..2, and
+// for tubes whether the partners are screened (ENS_SCREENED; bulk and slit
+// jobs always screen); ENS_RUNTIME: the modes are read from the job.
 constexpr int ENS_RUNTIME = -1;
-constexpr int ens_code(int tconstant, int pconstant, int confined) {
-  return (tconstant * 4 + pconstant) * 3 + confined;
+constexpr int ENS_SCREENED = 36;
+constexpr int ens_code(int tconstant, int pconstant, int confined, bool compact) {
+  return (tconstant * 4 + pconstant) * 3 + confined + (confined == 1 && compact ? ENS_SCREENED : 0);
 }
-constexpr int ens_tconstant(int code) { return code / 12; }
+constexpr int ens_tconstant(int code) { return code % ENS_SCREENED / 12; }
 constexpr int ens_pconstant(int code) { return (code / 3) % 4; }
 constexpr int ens_confined(int code) { return code % 3; }
+constexpr bool ens_compact(int code) { return ens_confined(code) != 1 || code >= ENS_SCREENED; }
 // Ensembles the resident kernels (single-job and batch) are also built for
 // with the modes fixed (FP32 pair math): Nose-Poincare thermostat with the
-// 1D barostat in a tube, the area barostat in a slit, the 3D barostat in
-// bulk.
-constexpr int ENS_TUBE_NP = ens_code(1, 2, 1);
-constexpr int ENS_SLIT_NP = ens_code(1, 3, 2);
-constexpr int ENS_BULK_NP = ens_code(1, 1, 0);
+// 1D barostat in a tube (narrow: every partner evaluated; wide: screened),
+// the area barostat in a slit, the 3D barostat in bulk.
+constexpr int ENS_TUBE_NP = ens_code(1, 2, 1, false);
+constexpr int ENS_WIDE_NP = ens_code(1, 2, 1, true);
+constexpr int ENS_SLIT_NP = ens_code(1, 3, 2, true);
+constexpr int ENS_BULK_NP = ens_code(1, 1, 0, true);
 
 // Resident path: molecules per energy block.  A replica's parts own whole
 // blocks, and the energy/virial totals are sums of block sums.
@@ -159,6 +163,7 @@ struct LaunchArgs {
                                 // bits: arrivals; high 32: XCD histogram of the parts)
   unsigned *abort;              // resident path, parts > 1: abort word, zeroed
   int same_xcd_ok;              // resident path: may use the same-XCD group barrier
+  int lds = 0;                  // global-state path: bytes of dynamic LDS of the launch
   int same_xcd_mode;            // same-XCD barrier: bit 0 agent-scope release, bit 1 agent-scope
                                 // acquire (else: stores drained to L2 / device-scope loads)
 };

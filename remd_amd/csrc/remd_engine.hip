@@ -79,11 +79,18 @@ int lds_bytes_host(int nmol, int nsite, int prec, int nt, bool grec) {
 }
 }  // namespace remd
 
+// LDS of a global-state launch: the layout, and up to 32 screening mask
+// words per lane (1024 partners of an item at a time) where they fit.
+static int lds_with_masks(int base, int nt, int lim) {
+  return base + std::max(0, std::min(16, (lim - base) / (8 * nt))) * 8 * nt;
+}
+
 // Bytes of one replica's site records (FP32 or FP64 site positions and
-// body-frame offsets, src/remdgpu.cu:2607-2651 layout stride).
+// body-frame offsets, src/remdgpu.cu:2607-2651 layout stride), whole
+// 16-byte vectors.
 static size_t rec_bytes(int nmol, int nsite, int prec) {
   const int stride = (nsite == 5) ? 18 : (nsite == 4 ? 16 : 12);
-  return (size_t)nmol * stride * (prec ? 8 : 4);
+  return ((size_t)nmol * stride * (prec ? 8 : 4) + 15) / 16 * 16;
 }
 
 static int device_lds_limit() {
@@ -259,6 +266,29 @@ static int validate(const remd_gpu_desc *d, const remd_gpu_scalars *sc) {
   return 0;
 }
 
+// Share of a molecule's window partners inside the cutoff, for molecules
+// spread evenly over a tube's accessible radius R - 2.8 A: the mean over two
+// radii and the angle between them of the cutoff's half-chord over the
+// window's half-length.
+static double tube_inside_fraction(const remd_gpu_desc *d) {
+  const double a = std::max(0.5, d->wall_length - 2.8);
+  const int n = 16;
+  double sum = 0.0;
+  for (int i = 0; i < n; i++)
+    for (int j = 0; j < n; j++)
+      for (int k = 0; k < n; k++) {
+        const double r1 = a * std::sqrt((i + 0.5) / n), r2 = a * std::sqrt((j + 0.5) / n);
+        const double rho2 = r1 * r1 + r2 * r2 - 2.0 * r1 * r2 * std::cos(M_PI * (k + 0.5) / n);
+        sum += std::sqrt(std::max(0.0, d->rcut * d->rcut - rho2));
+      }
+  return sum / (n * n * n) / (d->rcut + d->margin);
+}
+// Tubes whose windows hold a smaller share than this screen their partners
+// (R above about 10.4 A at a 9 A cutoff).  Interval without / with
+// screening, TIP4P, 40 A: R = 9 1.88 / 1.95 ms, 10 2.89 / 2.85, 11 3.43 /
+// 3.28, 12 4.46 / 4.00, 14 7.90 / 5.95; TIP5P: 10 3.18 / 3.22, 11 4.14 / 3.97.
+constexpr double TUBE_SCREEN_BELOW = 0.5;
+
 static void fill_params(const remd_gpu_desc *d, JobParams &J) {
   memset(&J, 0, sizeof(J));
   J.nmol = d->nmol;
@@ -274,9 +304,10 @@ static void fill_params(const remd_gpu_desc *d, JobParams &J) {
   J.sort_interval = d->sort_interval;
   J.nfwall = d->nfwall;
   J.precision = d->precision;
-  // bulk and slit windows are slabs of the box, mostly beyond the cutoff:
-  // screen the partners first; tube windows are mostly inside it
-  J.compact = d->confined == 1 ? 0 : 1;
+  // bulk and slit windows are slabs of the box, mostly beyond the cutoff, as
+  // are the windows of wide tubes: screen the partners first; narrow tubes'
+  // windows are mostly inside it
+  J.compact = d->confined == 1 ? tube_inside_fraction(d) < TUBE_SCREEN_BELOW : 1;
   // the rank sort's O(N^2 / threads) comparisons lose to the radix sort's
   // 16 passes from about this size (measured); REMD_SORT_RADIX_MIN overrides
   {
@@ -458,7 +489,7 @@ static int pick_parts(int capacity, int nrep, int N) {
 
 // Ensemble code of the job (selects the resident-kernel instantiation).
 static int job_ens(const remd_gpu *g) {
-  return g->prm.ens_fixed ? ens_code(g->prm.tmode, g->prm.pmode, g->prm.cmode) : ENS_RUNTIME;
+  return g->prm.ens_fixed ? ens_code(g->prm.tmode, g->prm.pmode, g->prm.cmode, g->prm.compact != 0) : ENS_RUNTIME;
 }
 
 // A resident-path launch of nrep replicas with a.parts workgroups each: the
@@ -637,6 +668,7 @@ extern "C" int remd_gpu_create(remd_gpu **out, const remd_gpu_desc *d, const rem
       return fail(REMD_EINVAL, "replica too large for workgroup LDS (" + std::to_string(g->lds) + " > " +
                                    std::to_string(lim) + " bytes)");
     }
+    g->lds = lds_with_masks(g->lds, g->nt, lim);
   }
 #define CK(...)                        \
   do {                                 \
@@ -1032,8 +1064,9 @@ extern "C" int remd_gpu_autotune(remd_gpu *g, int reps) {
   const int lim = device_lds_limit();
   for (int a = 0; a < 3; a++) {
     for (int C = 1; C <= 16; C *= 2) {
-      const int lds = lds_bytes_host(g->N, g->NS, g->prm.precision, nts[a], g->grec);
+      int lds = lds_bytes_host(g->N, g->NS, g->prm.precision, nts[a], g->grec);
       if (lds > lim) continue;
+      lds = lds_with_masks(lds, nts[a], lim);
       g->nt = nts[a];
       g->lds = lds;
       g->prm.chunks = C;
@@ -1056,7 +1089,7 @@ extern "C" int remd_gpu_autotune(remd_gpu *g, int reps) {
   }
   g->nt = bnt;
   g->prm.chunks = bc;
-  g->lds = lds_bytes_host(g->N, g->NS, g->prm.precision, bnt, g->grec);
+  g->lds = lds_with_masks(lds_bytes_host(g->N, g->NS, g->prm.precision, bnt, g->grec), bnt, lim);
   HIPCHK(hipMemcpyAsync(g->d_job, &g->prm, sizeof(JobParams), hipMemcpyHostToDevice, g->stream));
   // restore the force/energies of the resident state for the chosen shape
   int rc = launch(g, MODE_FORCE, 1, g->prm.margin, g->d_reps, g->nrep, false);

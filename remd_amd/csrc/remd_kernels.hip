@@ -95,6 +95,21 @@ template <int EM>
 __device__ __host__ constexpr int per_mask_of() {
   return EM < 0 ? -1 : (ens_confined(EM) == 1 ? 4 : (ens_confined(EM) == 2 ? 3 : 7));
 }
+// Layout of the site records: one contiguous record per molecule for narrow
+// tubes, where every partner is evaluated and the lanes of a wave share 16
+// or so neighbouring partners (the record's words then sit at constant
+// offsets of one address: 144 TIP4P, 2 to 4 % less per interval than with
+// planes), planes (Rec) elsewhere.
+template <int EM>
+__device__ __host__ constexpr bool records_of() {
+  return EM == ENS_TUBE_NP;
+}
+// bulk, slit and wide-tube jobs screen the partners
+template <int EM>
+__device__ __forceinline__ bool compact_of(JRef J) {
+  if constexpr (EM < 0) return J.compact != 0;
+  else return ens_compact(EM);
+}
 // the sort axis follows the confinement: x for the slit, z otherwise
 template <int EM>
 __device__ __forceinline__ int sort_axis_of(JRef J) {
@@ -123,11 +138,29 @@ __device__ __forceinline__ int sort_axis_of(JRef J) {
 #endif
 
 // ------------------------------------------------------------ LDS layout
-template <int NS>
+// Site records: COM (3) + NS sites x 3 words per molecule, padded to
+// STRIDE words and stored as planes of 16-byte vectors (the last plane of
+// the 5-site FP32 record is 8 bytes wide): lanes that read neighbouring
+// molecules read neighbouring vectors, so the screening and the record
+// writes meet no LDS bank conflict.  A record of its own per molecule (64
+// bytes for 4 sites) puts every lane's word on the same 4 of 64 banks.
+template <int NS, typename PT>
 struct Rec {
-  // COM (3) + NS sites x 3, padded for 8/16-byte LDS reads
   static constexpr int STRIDE = (NS == 5) ? 18 : (NS == 4 ? 16 : 12);
+  static constexpr int LEN = 3 + 3 * NS;                 // words in use
+  static constexpr int VW = 16 / (int)sizeof(PT);        // words of a full vector
+  static constexpr int FULL = STRIDE / VW;               // full planes
+  static constexpr int REST = STRIDE - FULL * VW;        // words of the narrow plane (0 or 2)
 };
+template <int W, typename PT>
+struct alignas(W * sizeof(PT)) RecVec {
+  PT v[W];
+};
+template <int W, typename PT>
+__device__ __forceinline__ RecVec<W, PT> rec_vec(const PT *rec, int N, int plane, int j) {
+  constexpr int VW = 16 / (int)sizeof(PT);
+  return *(const RecVec<W, PT> *)(rec + (size_t)plane * VW * N + (size_t)j * W);
+}
 
 __host__ __device__ inline int align16(int x) { return (x + 15) & ~15; }
 
@@ -142,16 +175,31 @@ __host__ __device__ inline int lds_bytes(int nmol, int nsite, int prec, int nt, 
   return region0 + win + align16(misc);
 }
 
+// LDS scratch for the screened partners of the work items: `words` 32-partner
+// bit masks per lane (even; 0: none, one word is then kept in a register).
+// Words 2 s and 2 s + 1 of lane t share the 8-byte slot s * NT + t, the slot
+// of the lane's own pair partial s on the resident path, so that a lane that
+// is done may write its partials while others still read their masks.
+struct MaskBuf {
+  unsigned *buf;
+  int words;
+};
+template <int NT>
+__device__ __forceinline__ unsigned *mask_word(const MaskBuf &mb, int w) {
+  return mb.buf + 2 * ((w >> 1) * NT + (int)threadIdx.x) + (w & 1);
+}
+
 struct Lds {
   char *region0;
   char *rec;     // site records: region 0, or global memory (grec)
   uint16_t *js, *je;
   double *red;   // NW x 32 doubles
   int *cnt;      // radix counts
+  MaskBuf mask;  // what the launch's LDS leaves
 };
 
 template <int NT>
-__device__ inline Lds lds_carve(char *smem, int nmol, int nsite, int prec, char *grec = nullptr) {
+__device__ inline Lds lds_carve(char *smem, int nmol, int nsite, int prec, int lds, char *grec) {
   const int stride = (nsite == 5) ? 18 : (nsite == 4 ? 16 : 12);
   const int rec = grec ? 0 : nmol * stride * (prec ? 8 : 4);
   const int sortb = 20 * nmol;
@@ -164,6 +212,9 @@ __device__ inline Lds lds_carve(char *smem, int nmol, int nsite, int prec, char 
   char *misc = smem + region0 + align16(4 * nmol);
   L.red = (double *)misc;
   L.cnt = (int *)(misc + (NT / WAVE) * 32 * 8);
+  const int base = lds_bytes(nmol, nsite, prec, NT, grec != nullptr);
+  L.mask.buf = (unsigned *)(smem + base);
+  L.mask.words = lds > base ? (lds - base) / (8 * NT) * 2 : 0;
   return L;
 }
 
@@ -815,6 +866,25 @@ struct PairK {
   PT L[3], Li[3];  // L: the box length on periodic axes, 0 on the others (no wrap there)
 };
 
+// Keeps the pair constants in vector registers: the step loop's scalar
+// registers are full, and a constant spilled from them is read back lane by
+// lane inside the pair loop (144 TIP4P tube: 1.330 ms per interval against
+// 1.345).
+template <int NS>
+__device__ __forceinline__ void vector_constants(PairK<NS, float> &k) {
+  asm("" : "+v"(k.rc), "+v"(k.rl), "+v"(k.rc2), "+v"(k.rl2), "+v"(k.coef), "+v"(k.coef30), "+v"(k.rs2));
+  asm("" : "+v"(k.sig2), "+v"(k.eps4), "+v"(k.eps48));
+#pragma unroll
+  for (int a = 0; a < NS; a++)
+#pragma unroll
+    for (int b = a; b < NS; b++) {
+      asm("" : "+v"(k.qq[a][b]));
+      k.qq[b][a] = k.qq[a][b];
+    }
+#pragma unroll
+  for (int d = 0; d < 3; d++) asm("" : "+v"(k.L[d]), "+v"(k.Li[d]));
+}
+
 template <int NS, typename AT = double>
 struct Acc {
   AT site[NS][3];
@@ -932,93 +1002,171 @@ __device__ __forceinline__ void pair_acc(const PT *gi, const PT (&ai)[NS][3], co
   acc.clmb += (AT)(sw * ecl);
 }
 
-template <int NS, typename PT>
-__device__ __forceinline__ void load_rec(PT (&r)[3 + 3 * NS], const PT *src) {
+// Record of molecule j.
+template <int NS, typename PT, bool RECORDS = false>
+__device__ __forceinline__ void load_rec(PT (&r)[3 + 3 * NS], const PT *rec, int N, int j) {
+  using R = Rec<NS, PT>;
+  if constexpr (RECORDS) {
 #pragma unroll
-  for (int u = 0; u < 3 + 3 * NS; u++) r[u] = src[u];
+    for (int u = 0; u < R::LEN; u++) r[u] = rec[j * R::STRIDE + u];
+    return;
+  }
+#pragma unroll
+  for (int p = 0; p < R::FULL; p++) {
+    const auto x = rec_vec<R::VW, PT>(rec, N, p, j);
+#pragma unroll
+    for (int u = 0; u < R::VW; u++)
+      if (p * R::VW + u < R::LEN) r[p * R::VW + u] = x.v[u];
+  }
+  if constexpr (R::REST != 0) {
+    const auto x = rec_vec<R::REST, PT>(rec, N, R::FULL, j);
+#pragma unroll
+    for (int u = 0; u < R::REST; u++) r[R::FULL * R::VW + u] = x.v[u];
+  }
+}
+
+// COM of molecule j.
+template <typename PT>
+__device__ __forceinline__ void load_com(PT (&c)[3], const PT *rec, int N, int j) {
+  constexpr int VW = 16 / (int)sizeof(PT);
+  const auto x = rec_vec<VW, PT>(rec, N, 0, j);
+  c[0] = x.v[0];
+  c[1] = x.v[1];
+  if constexpr (VW == 4) c[2] = x.v[2];
+  else c[2] = rec_vec<VW, PT>(rec, N, 1, j).v[0];
+}
+
+// |COM difference| on axis d reduced to the nearest image, for screening
+// only (the sign is lost and the rounding is not min_image's): both
+// coordinates lie in the box, so |x| < L; on the non-periodic axes L = 0 and
+// the minimum is -|x|.
+template <int PER, int NS, typename PT>
+__device__ __forceinline__ PT near_image(PT x, const PairK<NS, PT> &k, int d) {
+  const PT a = fabs(x);
+  if constexpr (PER < 0) return fmin(a, k.L[d] - a);
+  else return ((PER >> d) & 1) ? fmin(a, k.L[d] - a) : x;
+}
+
+// Screening of `n` <= 32 partners jj, jj + C, ... of a work item by COM
+// distance, radius slightly above the cutoff (pair_acc decides): bit u of
+// the result is partner u; molecule i itself passes.  The COMs are loaded
+// SCREEN_BATCH at a time, so that a lone wave waits for LDS once a batch,
+// not once a partner (one ahead: about 380 cycles a partner, 1820 TIP4P).
+constexpr int SCREEN_BATCH = 8;
+template <int NS, typename PT, int PER>
+__device__ __forceinline__ unsigned screen(const PT *rec, int N, int jj, int C, int n, const PT *gi,
+                                           const PairK<NS, PT> &k) {
+  unsigned mask = 0u;
+  const unsigned last = (unsigned)(jj + (n - 1) * C);
+  for (int u0 = 0; u0 < n; u0 += SCREEN_BATCH) {
+    PT c[SCREEN_BATCH][3];
+#pragma unroll
+    for (int u = 0; u < SCREEN_BATCH; u++) {
+      // partners beyond the last one repeat it; j mod N for j < 2 N
+      const unsigned x = min((unsigned)(jj + (u0 + u) * C), last);
+      load_com(c[u], rec, N, (int)min(x, x - (unsigned)N));
+    }
+    unsigned m = 0u;
+#pragma unroll
+    for (int u = 0; u < SCREEN_BATCH; u++) {
+      PT dg[3];
+#pragma unroll
+      for (int d = 0; d < 3; d++) dg[d] = near_image<PER>(gi[d] - c[u][d], k, d);
+      const PT r2 = dg[0] * dg[0] + dg[1] * dg[1] + dg[2] * dg[2];
+      m |= (r2 < k.rs2 ? 1u : 0u) << u;
+    }
+    mask |= m << u0;
+  }
+  return n < 32 ? mask & ((1u << n) - 1u) : mask;
 }
 
 // The partners of work item (i, c): jj = js + c, js + c + C, ... <= je
 // (indices mod N), each through pair_acc, in this order.  The record of the
 // next partner is loaded while the current pair is computed.  With
-// `compact` the COM distances of the next 32 partners are screened first
-// (radius slightly above the cutoff) and only the ones inside go through
-// pair_acc, still in order: the same pairs and the same sums, with less
-// work where most partners lie beyond the cutoff (bulk and slit windows).
-template <int NS, int QB, typename PT, int PER, typename AT>
+// `compact` the partners are screened first and only the ones inside go
+// through pair_acc, still in order: the same pairs and the same sums, with
+// less work where most partners lie beyond the cutoff.  The screening leaves
+// bit masks in LDS (32 partners a word, as many words as fit), so that every
+// lane then walks its own list without a break: a wave runs as many pair
+// steps as its longest list, not the sum of its longest 32-partner pieces
+// (1820 TIP4P bulk: 110 steps instead of 201 for lists of 100 on average;
+// 512 TIP5P slit 81 instead of 97 for 74).  Pair pass of a step: 1820 TIP4P
+// 283 -> 114 us, 1374 TIP5P slit 310 -> 172 us, 512 TIP5P slit 94 -> 57 us;
+// the pair loop is then at the FP32 issue rate of its one wave per SIMD.
+// Both loops are wave-uniform: a lane past its last partner takes the
+// molecule itself, which adds nothing.
+template <int NT, int NS, int QB, typename PT, int PER, bool RECORDS, typename AT>
 __device__ __forceinline__ void pair_window_run(const PT *rec, int N, int i, int js, int je, int c0, int C,
                                                 bool compact, const PT *gi, const PT (&ai)[NS][3],
-                                                const PairK<NS, PT> &k, Acc<NS, AT> &acc) {
-  constexpr int ST = Rec<NS>::STRIDE;
+                                                const PairK<NS, PT> &k, const MaskBuf &mb, Acc<NS, AT> &acc) {
   constexpr int RL = 3 + 3 * NS;
   if (!compact) {
     int jj = js + c0;
-    if (jj > je) return;
-    int j = (jj >= N) ? jj - N : jj;
-    PT rj[RL];
-    load_rec<NS, PT>(rj, rec + j * ST);
+    // two records in turn (no copies between them); a lane past its last
+    // partner takes itself, which adds nothing, so the loop is wave-uniform
+    auto fetch = [&](PT (&r)[RL], int &j) {
+      const bool on = jj <= je;
+      j = on ? ((jj >= N) ? jj - N : jj) : i;
+      jj += C;
+      load_rec<NS, PT, RECORDS>(r, rec, N, j);
+      return __any(on);
+    };
+    PT ra[RL], rb[RL];
+    int ja, jb;
+    if (!fetch(ra, ja)) return;
     for (;;) {
-      const int jn = jj + C;
-      const bool more = jn <= je;
-      const int jx = more ? ((jn >= N) ? jn - N : jn) : j;
-      PT rn[RL];
-      load_rec<NS, PT>(rn, rec + jx * ST);
-      pair_acc<NS, QB, PT, PER>(gi, ai, rj, k, j == i, acc);
-      if (!more) break;
-      jj = jn;
-      j = jx;
-#pragma unroll
-      for (int u = 0; u < RL; u++) rj[u] = rn[u];
+      const bool more_b = fetch(rb, jb);
+      pair_acc<NS, QB, PT, PER>(gi, ai, ra, k, ja == i, acc);
+      if (!more_b) break;
+      const bool more_a = fetch(ra, ja);
+      pair_acc<NS, QB, PT, PER>(gi, ai, rb, k, jb == i, acc);
+      if (!more_a) break;
     }
     return;
   }
-  for (int base = js + c0; base <= je; base += 32 * C) {
+  int left = js + c0 <= je ? (je - js - c0) / C + 1 : 0;  // partners not screened yet
+  // i itself as a partner: position `self` in the item's list, if any
+  int self = i - (js + c0);
+  self = self < 0 ? self + N : self;
+  self = self % C == 0 ? self / C : -1;
+  for (int base = js + c0; left > 0;) {
+    const int part = min(left, mb.words ? 32 * mb.words : 32);
+    const int nw = (part + 31) >> 5;
+    unsigned m0 = 0u;
+    for (int w = 0; w < nw; w++) {
+      m0 = screen<NS, PT, PER>(rec, N, base + 32 * w * C, C, min(32, part - 32 * w), gi, k);
+      if ((self >> 5) == w) m0 &= ~(1u << (self & 31));
+      if (mb.words) *mask_word<NT>(mb, w) = m0;
+    }
+    // the next partner's record, or the molecule's own (which adds nothing)
+    // where the current word is spent
+    int w = 0, b0 = base - 32 * C;
     unsigned mask = 0u;
-    {
-      int jj = base;
-      int j = (jj >= N) ? jj - N : jj;
-      PT c[3] = {rec[j * ST], rec[j * ST + 1], rec[j * ST + 2]};
-      for (int u = 0; u < 32; u++) {
-        const int jn = jj + C;
-        const bool more = u < 31 && jn <= je;
-        const int jx = more ? ((jn >= N) ? jn - N : jn) : j;
-        const PT cn[3] = {rec[jx * ST], rec[jx * ST + 1], rec[jx * ST + 2]};
-        PT dg[3];
-#pragma unroll
-        for (int d = 0; d < 3; d++) dg[d] = min_image<PER>(gi[d] - c[d], k, d);
-        const PT r2 = dg[0] * dg[0] + dg[1] * dg[1] + dg[2] * dg[2];
-        if (j != i && r2 < k.rs2) mask |= 1u << u;
-        if (!more) break;
-        jj = jn;
-        j = jx;
-        c[0] = cn[0];
-        c[1] = cn[1];
-        c[2] = cn[2];
+    auto fetch = [&](PT (&r)[RL], bool &none) {
+      if (mask == 0u && w < nw) {
+        mask = mb.words ? *mask_word<NT>(mb, w) : m0;
+        w++;
+        b0 += 32 * C;
       }
-    }
-    if (!mask) continue;
-    int u = __builtin_ctz(mask);
-    mask &= mask - 1u;
-    int j = base + u * C;
-    j = (j >= N) ? j - N : j;
-    PT rj[RL];
-    load_rec<NS, PT>(rj, rec + j * ST);
-    for (;;) {
-      const bool more = mask != 0u;
-      int jx = j;
-      if (more) {
-        jx = base + __builtin_ctz(mask) * C;
-        jx = (jx >= N) ? jx - N : jx;
-        mask &= mask - 1u;
-      }
-      PT rn[RL];
-      load_rec<NS, PT>(rn, rec + jx * ST);
-      pair_acc<NS, QB, PT, PER>(gi, ai, rj, k, false, acc);
+      none = mask == 0u;
+      const int jj = b0 + (none ? 0 : __builtin_ctz(mask)) * C;
+      load_rec<NS, PT>(r, rec, N, none ? i : ((jj >= N) ? jj - N : jj));
+      mask &= mask - 1u;
+      return __any(!none || w < nw);
+    };
+    PT ra[RL], rb[RL];
+    bool na, nb;
+    bool more = fetch(ra, na);
+    while (more) {
+      more = fetch(rb, nb);
+      pair_acc<NS, QB, PT, PER>(gi, ai, ra, k, na, acc);
       if (!more) break;
-      j = jx;
-#pragma unroll
-      for (int v = 0; v < RL; v++) rj[v] = rn[v];
+      more = fetch(ra, na);
+      pair_acc<NS, QB, PT, PER>(gi, ai, rb, k, nb, acc);
     }
+    left -= part;
+    base += part * C;
+    self -= part;
   }
 }
 
@@ -1027,10 +1175,10 @@ __device__ __forceinline__ void pair_window_run(const PT *rec, int N, int i, int
 // pair math sums in FP64.  The chunks are then reduced in FP64.  A chunk's
 // partners do not depend on how a replica is split over workgroups, so the
 // results stay the same bits for any split.
-template <int NS, int QB, typename PT, int PER = -1>
+template <int NT, int NS, int QB, typename PT, int PER = -1, bool RECORDS = false>
 __device__ __forceinline__ void pair_window(const PT *rec, int N, int i, int js, int je, int c0, int C,
                                             bool compact, const PT *gi, const PT (&ai)[NS][3],
-                                            const PairK<NS, PT> &k, Acc<NS> &acc) {
+                                            const PairK<NS, PT> &k, const MaskBuf &mb, Acc<NS> &acc) {
   if constexpr (sizeof(PT) == 4) {
     Acc<NS, float> part;
 #pragma unroll
@@ -1038,7 +1186,7 @@ __device__ __forceinline__ void pair_window(const PT *rec, int N, int i, int js,
     part.corr[0] = part.corr[1] = part.corr[2] = 0.0f;
     part.vir[0] = part.vir[1] = part.vir[2] = 0.0f;
     part.lj = part.clmb = 0.0f;
-    pair_window_run<NS, QB, PT, PER>(rec, N, i, js, je, c0, C, compact, gi, ai, k, part);
+    pair_window_run<NT, NS, QB, PT, PER, RECORDS>(rec, N, i, js, je, c0, C, compact, gi, ai, k, mb, part);
 #pragma unroll
     for (int a = 0; a < NS; a++)
 #pragma unroll
@@ -1051,16 +1199,16 @@ __device__ __forceinline__ void pair_window(const PT *rec, int N, int i, int js,
     acc.lj = (double)part.lj;
     acc.clmb = (double)part.clmb;
   } else {
-    pair_window_run<NS, QB, PT, PER>(rec, N, i, js, je, c0, C, compact, gi, ai, k, acc);
+    pair_window_run<NT, NS, QB, PT, PER, RECORDS>(rec, N, i, js, je, c0, C, compact, gi, ai, k, mb, acc);
   }
 }
 
-// M2A: LDS records (COM centred on the box, site offsets R(q) b).
-template <int NT, int NS, typename PT>
+// M2A: site records (COM centred on the box, site offsets R(q) b).
+template <int NT, int NS, typename PT, bool RECORDS = false>
 __device__ void m2a(JRef J, const double *mol, int N, double L0, double L1, double L2, PT *rec) {
-  constexpr int ST = Rec<NS>::STRIDE;
+  using R = Rec<NS, PT>;
   for (int i = threadIdx.x; i < N; i += NT) {
-    PT *o = rec + i * ST;
+    PT o[R::STRIDE];
     o[0] = (PT)((mol[F_RX * N + i] - 0.5) * L0);
     o[1] = (PT)((mol[F_RY * N + i] - 0.5) * L1);
     o[2] = (PT)((mol[F_RZ * N + i] - 0.5) * L2);
@@ -1073,6 +1221,26 @@ __device__ void m2a(JRef J, const double *mol, int N, double L0, double L1, doub
       o[4 + 3 * a] = (PT)t[1];
       o[5 + 3 * a] = (PT)t[2];
     }
+    if constexpr (RECORDS) {
+#pragma unroll
+      for (int u = 0; u < R::LEN; u++) rec[i * R::STRIDE + u] = o[u];
+      continue;
+    }
+#pragma unroll
+    for (int u = R::LEN; u < R::STRIDE; u++) o[u] = PT(0);
+#pragma unroll
+    for (int p = 0; p < R::FULL; p++) {
+      RecVec<R::VW, PT> x;
+#pragma unroll
+      for (int u = 0; u < R::VW; u++) x.v[u] = o[p * R::VW + u];
+      *(RecVec<R::VW, PT> *)(rec + (size_t)p * R::VW * N + (size_t)i * R::VW) = x;
+    }
+    if constexpr (R::REST != 0) {
+      RecVec<R::REST, PT> x;
+#pragma unroll
+      for (int u = 0; u < R::REST; u++) x.v[u] = o[R::FULL * R::VW + u];
+      *(RecVec<R::REST, PT> *)(rec + (size_t)R::FULL * R::VW * N + (size_t)i * R::REST) = x;
+    }
   }
 }
 
@@ -1083,7 +1251,6 @@ __device__ void force_pass(JRef J, double *mol, int N, Sc &c, const Lds &S,
                            double *site_dbg, double *pt_sc) {
   PT_DECL
   constexpr int QB = (NS == 3) ? 0 : 1;
-  constexpr int ST = Rec<NS>::STRIDE;
   PT *rec = (PT *)S.rec;
   m2a<NT, NS, PT>(J, mol, N, c.L[0], c.L[1], c.L[2], rec);
   __syncthreads();
@@ -1128,6 +1295,7 @@ __device__ void force_pass(JRef J, double *mol, int N, Sc &c, const Lds &S,
     k.Li[d] = (PT)(1.0 / c.L[d]);
   }
 
+  const MaskBuf mb = S.mask;
   const int C = J.chunks;
   const int lc = __ffs(C) - 1;  // log2(C)
   double e_lj = 0.0, e_cl = 0.0, e_wall = 0.0, vir[3] = {0.0, 0.0, 0.0};
@@ -1147,7 +1315,8 @@ __device__ void force_pass(JRef J, double *mol, int N, Sc &c, const Lds &S,
     acc.vir[0] = acc.vir[1] = acc.vir[2] = 0.0;
     acc.lj = acc.clmb = 0.0;
     if (active) {
-      const PT *ri = rec + i * ST;
+      PT ri[3 + 3 * NS];
+      load_rec<NS, PT>(ri, rec, N, i);
       PT gi[3] = {ri[0], ri[1], ri[2]};
       PT ai[NS][3];
 #pragma unroll
@@ -1156,7 +1325,7 @@ __device__ void force_pass(JRef J, double *mol, int N, Sc &c, const Lds &S,
         ai[a][1] = ri[4 + 3 * a];
         ai[a][2] = ri[5 + 3 * a];
       }
-      pair_window<NS, QB, PT>(rec, N, i, S.js[i], S.je[i], cc, C, J.compact != 0, gi, ai, k, acc);
+      pair_window<NT, NS, QB, PT>(rec, N, i, S.js[i], S.je[i], cc, C, J.compact != 0, gi, ai, k, mb, acc);
     }
     // fixed xor butterfly over the C lanes of molecule i
     for (int m = 1; m < C; m <<= 1) {
@@ -1400,7 +1569,7 @@ __device__ void run_replica(const LaunchArgs &a, const DescD &R, JRef J, char *s
   const int N = J.nmol;
   double *mol = gen(R.mol);
   int *mid = gen(R.mid);
-  Lds S = lds_carve<NT>(smem, N, NS, J.precision, gen(R.grec));
+  Lds S = lds_carve<NT>(smem, N, NS, J.precision, a.lds, gen(R.grec));
   Sc c;
   load_sc(c, gen(R.sc));
 
@@ -1822,8 +1991,8 @@ __device__ void force_range(JRef J, double *mol, int N, const Sc &c, const LdsR 
   PT_DECL
   (void)pt_sc;
   constexpr int QB = (NS == 3) ? 0 : 1;
-  constexpr int ST = Rec<NS>::STRIDE;
   const PT *rec = (const PT *)S.region0;
+  const MaskBuf mb = {(unsigned *)S.part, 2 * (S.part_n / NT)};
   PairK<NS, PT> k;
   if (sizeof(PT) == 4) {
     k.rc = J.f_rc;
@@ -1862,6 +2031,7 @@ __device__ void force_range(JRef J, double *mol, int N, const Sc &c, const LdsR 
     k.L[d] = J.per[d] ? (PT)c.L[d] : PT(0);
     k.Li[d] = (PT)(1.0 / c.L[d]);
   }
+  if constexpr (sizeof(PT) == 4) vector_constants(k);
   const int C = J.chunks;
   const int B = (NT / C) / EB * EB;  // molecules per round, whole energy blocks
   const int NV = npart(NS, site_dbg != nullptr);
@@ -1906,7 +2076,8 @@ __device__ void force_range(JRef J, double *mol, int N, const Sc &c, const LdsR 
         f1 = J.fwall[2 * (widx + 1)];
         e1 = J.fwall[2 * (widx + 1) + 1];
       }
-      const PT *ri = rec + i * ST;
+      PT ri[3 + 3 * NS];
+      load_rec<NS, PT, records_of<EM>()>(ri, rec, N, i);
       PT gi[3] = {ri[0], ri[1], ri[2]};
       PT ai[NS][3];
 #pragma unroll
@@ -1915,8 +2086,8 @@ __device__ void force_range(JRef J, double *mol, int N, const Sc &c, const LdsR 
         ai[a][1] = ri[4 + 3 * a];
         ai[a][2] = ri[5 + 3 * a];
       }
-      pair_window<NS, QB, PT, per_mask_of<EM>()>(rec, N, i, S.js[i], S.je[i], cc, C, J.compact != 0, gi, ai, k,
-                                              acc);
+      pair_window<NT, NS, QB, PT, per_mask_of<EM>(), records_of<EM>()>(rec, N, i, S.js[i], S.je[i], cc, C, compact_of<EM>(J), gi,
+                                                     ai, k, mb, acc);
       double e_wall = 0.0;
       if (wall) {
         const double f = (f1 - f0) * dri * (wu - dr * widx) + f0;
@@ -2140,7 +2311,7 @@ __device__ bool forces_resident(JRef J, double *mol, int N, Sc &c, const LdsR &S
                                 int i0, int i1, double *site_dbg, double *pt_sc = nullptr) {
   PT_DECL
   (void)pt_sc;
-  m2a<NT, NS, PT>(J, mol, N, c.L[0], c.L[1], c.L[2], (PT *)S.region0);
+  m2a<NT, NS, PT, records_of<EM>()>(J, mol, N, c.L[0], c.L[1], c.L[2], (PT *)S.region0);
   __syncthreads();
   PT_MARK(4, pt_sc);
   const int nblk = (N + EB - 1) / EB;
@@ -2396,8 +2567,9 @@ __global__ __launch_bounds__(RNT) void resident_batch_kernel(LaunchArgs a) {
   g.xbuf = gen(R.xbuf);
   g.epoch = 0;
   const unsigned variant = (e >> 8) & 15u;
-  const int ens = J.ens_fixed ? ens_code(J.tmode, J.pmode, J.cmode) : ENS_RUNTIME;
+  const int ens = J.ens_fixed ? ens_code(J.tmode, J.pmode, J.cmode, J.compact != 0) : ENS_RUNTIME;
   if (ens == ENS_TUBE_NP && run_resident_fixed<ENS_TUBE_NP>(variant, a, R, J, smem, g)) return;
+  if (ens == ENS_WIDE_NP && run_resident_fixed<ENS_WIDE_NP>(variant, a, R, J, smem, g)) return;
   if (ens == ENS_SLIT_NP && run_resident_fixed<ENS_SLIT_NP>(variant, a, R, J, smem, g)) return;
   if (ens == ENS_BULK_NP && run_resident_fixed<ENS_BULK_NP>(variant, a, R, J, smem, g)) return;
   switch (variant) {
@@ -2716,6 +2888,7 @@ const void *resident_fn_fixed(int nsite, int ens) {
     if (nsite == 5) return (const void *)resident_kernel<RNT, 5, float, E>; \
   }
   REMD_RES_ENS(ENS_TUBE_NP)
+  REMD_RES_ENS(ENS_WIDE_NP)
   REMD_RES_ENS(ENS_SLIT_NP)
   REMD_RES_ENS(ENS_BULK_NP)
 #undef REMD_RES_ENS
@@ -2785,13 +2958,15 @@ hipError_t resident_occupancy(int nsite, int prec, int ens, int lds, int *per_cu
 
 hipError_t launch_interval(const LaunchArgs &a, int nt, int nsite, int prec, int lds, hipStream_t st) {
   if (a.nrep <= 0) return hipSuccess;
-  return launch_fn(interval_fn(nt, nsite, prec), a.nrep, nt, a, lds, st);
+  LaunchArgs arg = a;
+  arg.lds = lds;
+  return launch_fn(interval_fn(nt, nsite, prec), a.nrep, nt, arg, lds, st);
 }
 
 hipError_t set_kernel_lds_limit(int bytes) {
   hipError_t e = hipSuccess;
-  const int ens[4] = {ENS_RUNTIME, ENS_TUBE_NP, ENS_SLIT_NP, ENS_BULK_NP};
-  for (int k = 0; k < 4 && e == hipSuccess; k++)
+  const int ens[5] = {ENS_RUNTIME, ENS_TUBE_NP, ENS_WIDE_NP, ENS_SLIT_NP, ENS_BULK_NP};
+  for (int k = 0; k < 5 && e == hipSuccess; k++)
     for (int ns = 3; ns <= 5 && e == hipSuccess; ns++)
       for (int pr = 0; pr < 2 && e == hipSuccess; pr++)
         e = hipFuncSetAttribute(resident_fn(ns, pr, ens[k]), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
