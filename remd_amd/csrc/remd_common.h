@@ -94,10 +94,12 @@ struct ReplicaDesc {
   double *sc;                   // NSC doubles
   double *site_f;               // optional: nsite*nmol*3 (last force pass)
   int *win;                     // optional: 3*nmol window (js, je, whole-ring flag)
-  double *xbuf;                 // resident path with parts > 1: exchange rows (xbuf_parity_doubles)
-  double *gbuf;                 // split-global path: one private state copy per part (gm_part_doubles)
+  double *xbuf;                 // parts > 1: exchange rows (resident path: 2 x xbuf_parity_doubles,
+                                // global-state path: grow_doubles)
+  double *gbuf;                 // split-global path, and global-state path with parts > 1: one
+                                // private state copy per part (gm_part_doubles)
   void *grec;                   // global-state path, replicas whose site records do not fit the
-                                // LDS: the records in global memory (nmol x stride x FP32/FP64)
+                                // LDS: the records in global memory, one copy per part (rec_bytes)
 };
 
 // Resident path: threads per workgroup (4 waves: one per SIMD of a CU).
@@ -149,20 +151,36 @@ __host__ __device__ inline size_t gm_part_doubles(int nmol) {
   return (size_t)NFIELD * nmol + (size_t)6 * ((nmol + EB - 1) / EB) + (size_t)((nmol + 1) / 2);
 }
 
+// Site records of a replica (bytes): FP32 or FP64 words, whole 16-byte vectors.
+__host__ __device__ inline size_t rec_bytes(int nmol, int nsite, int prec) {
+  const int stride = (nsite == 5) ? 18 : (nsite == 4 ? 16 : 12);
+  return ((size_t)nmol * stride * (prec ? 8 : 4) + 15) / 16 * 16;
+}
+
+// Global-state path, replicas split over workgroups: values of a molecule's
+// exchange row (F[3], n[4], vir[3], lj, clmb, wall), value-major, and two
+// rows (step parity) per molecule.
+constexpr int GR = 13;
+__host__ __device__ inline size_t grow_doubles(int nmol) { return (size_t)2 * GR * nmol; }
+
+// Bit of a group word (arrivals count in its low half): the replica's state
+// has been written back.
+constexpr unsigned long long REPLICA_DONE = 1ull << 63;
+
 struct LaunchArgs {
   const ReplicaDesc *reps;
   int nrep;
   int mode;
   int do_sort;                  // MODE_FORCE only
   double margin;                // MODE_FORCE only
-  int parts;                    // resident path: workgroups per replica (blk == nullptr)
+  int parts;                    // workgroups per replica (blk == nullptr)
   const unsigned *blk = nullptr; // resident batch launch: per-workgroup entry (rep << 12 |
                                  // variant << 8 | parts << 4 | part), ~0u for an idle workgroup
   int nblk = 0;                  // workgroups of a resident batch launch
-  unsigned long long *sync;     // resident path, parts > 1: nrep group words, zeroed (low 32
-                                // bits: arrivals; high 32: XCD histogram of the parts)
-  unsigned *abort;              // resident path, parts > 1: abort word, zeroed
-  int same_xcd_ok;              // resident path: may use the same-XCD group barrier
+  unsigned long long *sync;     // parts > 1: nrep group words, zeroed
+  unsigned *abort;              // parts > 1: abort word, zeroed
+  int same_xcd_ok;              // parts > 1: may use the same-XCD group barrier
+  int skip_done = 0;            // global-state path: leave replicas with REPLICA_DONE alone
   int lds = 0;                  // global-state path: bytes of dynamic LDS of the launch
   int same_xcd_mode;            // same-XCD barrier: bit 0 agent-scope release, bit 1 agent-scope
                                 // acquire (else: stores drained to L2 / device-scope loads)

@@ -85,14 +85,6 @@ static int lds_with_masks(int base, int nt, int lim) {
   return base + std::max(0, std::min(16, (lim - base) / (8 * nt))) * 8 * nt;
 }
 
-// Bytes of one replica's site records (FP32 or FP64 site positions and
-// body-frame offsets, src/remdgpu.cu:2607-2651 layout stride), whole
-// 16-byte vectors.
-static size_t rec_bytes(int nmol, int nsite, int prec) {
-  const int stride = (nsite == 5) ? 18 : (nsite == 4 ? 16 : 12);
-  return ((size_t)nmol * stride * (prec ? 8 : 4) + 15) / 16 * 16;
-}
-
 static int device_lds_limit() {
   static int lim = -1;
   if (lim < 0) {
@@ -111,6 +103,7 @@ static int device_lds_limit() {
 // -------------------------------------------------------------- job
 // Largest number of workgroups one replica is split over (resident path).
 constexpr int GMAX = 8;
+constexpr int NXCD = 8;
 
 struct remd_gpu {
   remd_gpu_desc desc;
@@ -121,8 +114,9 @@ struct remd_gpu {
   bool resident = false;     // state in LDS for the launch (resident_kernel)
   bool gm = false;           // resident kernel, split-global variant: state in per-part global copies
   double *d_gbuf = nullptr;  // split-global: nrep x GMAX x gm_part_doubles(N)
-  char *d_grec = nullptr;    // global-state path: site records in global memory (rec_bytes each)
+  char *d_grec = nullptr;    // global-state path: site records in global memory (gparts x rec_bytes each)
   bool grec = false;         // the global-state path's site records do not fit the LDS
+  int gparts = 1;            // global-state path: most workgroups per replica
   unsigned *d_blk1 = nullptr;  // split-global: workgroup table of the last (nrep, parts) launch shape
   int blk1_nrep = 0, blk1_parts = 0, blk1_n = 0;
   int capacity = 0;          // resident workgroups the device holds at once
@@ -365,6 +359,20 @@ static void fill_params(const remd_gpu_desc *d, JobParams &J) {
   }
 }
 
+// Most workgroups per replica of a global-state launch of nrep replicas on a
+// device of ncu CUs: all of them resident at once, one per CU, the parts of
+// a replica on one XCD (block indices equal mod 8), and enough molecules for
+// a whole wave of work items per part.  100 steps of 8 replicas of 2048
+// TIP4P: 71.0 ms on 8 workgroups, 18.6 ms on 64.  Below GLOBAL_SPLIT_MIN
+// (jobs that ask for this path) one workgroup per replica as before.
+constexpr int GLOBAL_SPLIT_MIN = 512;
+static int global_parts_max(int ncu, int nrep, int nmol, int chunks) {
+  if (nmol < GLOBAL_SPLIT_MIN || nrep < 1) return 1;
+  const int rows = (nrep + NXCD - 1) / NXCD;
+  const int p = std::min(std::min(GMAX, ncu / (NXCD * rows)), nmol * std::max(1, chunks) / 64);
+  return std::max(1, p);
+}
+
 extern "C" size_t remd_gpu_footprint(const remd_gpu_desc *d) {
   if (!d) return 0;
   const size_t N = (size_t)d->nmol, R = (size_t)d->nreplica;
@@ -376,8 +384,11 @@ extern "C" size_t remd_gpu_footprint(const remd_gpu_desc *d) {
   b += R * 2 * xbuf_parity_doubles((int)N) * sizeof(double) + (R + 1) * sizeof(unsigned long long);
   // split-global private copies (replicas of 512 or more molecules may take that path)
   if (N >= 512) b += R * GMAX * gm_part_doubles((int)N) * sizeof(double);
-  // global-state path site records in global memory (replicas beyond the LDS)
-  if (N >= 1024) b += R * rec_bytes((int)N, d->nsite, d->precision);
+  // global-state path site records in global memory (replicas beyond the
+  // LDS) and exchange rows, for every workgroup of a replica
+  const size_t G = (size_t)global_parts_max(256, d->nreplica, d->nmol, 1);
+  if (N >= 1024) b += R * G * rec_bytes((int)N, d->nsite, d->precision);
+  if (N >= GLOBAL_SPLIT_MIN) b += R * grow_doubles((int)N) * sizeof(double);
   return b;
 }
 
@@ -442,9 +453,11 @@ static void refresh_reps(remd_gpu *g) {
     R.sc = g->d_sc + (size_t)r * NSC;
     R.site_f = g->debug ? g->d_site + (size_t)r * g->N * g->NS * 3 : nullptr;
     R.win = g->debug ? g->d_win + (size_t)r * g->N * 3 : nullptr;
-    R.xbuf = g->d_xbuf ? g->d_xbuf + (size_t)r * 2 * xbuf_parity_doubles(g->N) : nullptr;
-    R.gbuf = g->d_gbuf ? g->d_gbuf + (size_t)r * GMAX * gm_part_doubles(g->N) : nullptr;
-    R.grec = g->d_grec ? (void *)(g->d_grec + (size_t)r * rec_bytes(g->N, g->NS, g->prm.precision)) : nullptr;
+    const size_t xrows = g->resident ? 2 * xbuf_parity_doubles(g->N) : grow_doubles(g->N);
+    R.xbuf = g->d_xbuf ? g->d_xbuf + (size_t)r * xrows : nullptr;
+    R.gbuf = g->d_gbuf ? g->d_gbuf + (size_t)r * (g->resident ? GMAX : g->gparts) * gm_part_doubles(g->N) : nullptr;
+    R.grec = g->d_grec ? (void *)(g->d_grec + (size_t)r * g->gparts * rec_bytes(g->N, g->NS, g->prm.precision))
+                       : nullptr;
   }
 }
 
@@ -533,6 +546,35 @@ static int launch_res(remd_gpu *g, LaunchArgs &a, hipStream_t st) {
   return 0;
 }
 
+// A global-state launch of a.nrep replicas (from group word a.sync) over up
+// to gparts workgroups each.  A launch whose parts could not all be resident
+// (other work held the device) is completed by one workgroup per replica:
+// the replicas that had finished are left alone, the others start from
+// their state, which an aborted part does not touch.  Same bits either way.
+static int launch_global(remd_gpu *g, LaunchArgs &a, hipStream_t st) {
+  a.parts = g->gparts;
+  if (a.parts > 1) {
+    HIPCHK(hipMemsetAsync(a.sync, 0, sizeof(unsigned long long) * a.nrep, st));
+    // REMD_GLOBAL_ABORT=1 (tests): the abort word starts set, so parts that
+    // wait long enough to look at it give up and the completion below runs
+    const char *e = std::getenv("REMD_GLOBAL_ABORT");
+    HIPCHK(hipMemsetAsync(a.abort, e && e[0] == '1' ? 1 : 0, sizeof(unsigned long long), st));
+  }
+  HIPCHK(launch_interval(a, g->nt, g->NS, g->prm.precision, g->lds, st));
+  if (a.parts > 1) {
+    HIPCHK(hipMemcpyAsync(g->h_abort, a.abort, sizeof(unsigned), hipMemcpyDeviceToHost, st));
+    HIPCHK(hipStreamSynchronize(st));
+    if (*g->h_abort != 0u) {
+      *g->h_abort = 0u;
+      a.parts = 1;
+      a.skip_done = 1;
+      HIPCHK(launch_interval(a, g->nt, g->NS, g->prm.precision, g->lds, st));
+      a.skip_done = 0;
+    }
+  }
+  return 0;
+}
+
 static int launch(remd_gpu *g, int mode, int do_sort, double margin, const ReplicaDesc *reps, int nrep,
                   bool timed) {
   LaunchArgs a;
@@ -556,10 +598,12 @@ static int launch(remd_gpu *g, int mode, int do_sort, double margin, const Repli
     int rc = launch_res(g, a, g->stream);
     if (rc) return rc;
   } else {
-    HIPCHK(launch_interval(a, g->nt, g->NS, g->prm.precision, g->lds, g->stream));
+    int rc = launch_global(g, a, g->stream);
+    if (rc) return rc;
+    g->last_parts = a.parts;
   }
   if (timed) HIPCHK(hipEventRecord(g->ev1, g->stream));
-  if (a.parts > 1)
+  if (g->resident && a.parts > 1)
     HIPCHK(hipMemcpyAsync(g->h_abort, a.abort, sizeof(unsigned), hipMemcpyDeviceToHost, g->stream));
   return 0;
 }
@@ -568,7 +612,7 @@ static int launch(remd_gpu *g, int mode, int do_sort, double margin, const Repli
 // not all be resident gives up (no state is written back) instead of waiting.
 static int finish(remd_gpu *g) {
   HIPCHK(hipStreamSynchronize(g->stream));
-  if (g->last_parts > 1 && *g->h_abort != 0u) {
+  if (g->resident && g->last_parts > 1 && *g->h_abort != 0u) {
     *g->h_abort = 0u;
     return fail(REMD_EHIP, "resident launch aborted: the parts of a replica were not co-resident "
                            "(another kernel held the device)");
@@ -669,6 +713,10 @@ extern "C" int remd_gpu_create(remd_gpu **out, const remd_gpu_desc *d, const rem
                                    std::to_string(lim) + " bytes)");
     }
     g->lds = lds_with_masks(g->lds, g->nt, lim);
+    int dev = 0, ncu = 0;
+    hipGetDevice(&dev);
+    if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess)
+      g->gparts = global_parts_max(ncu, g->nrep, g->N, g->prm.chunks);
   }
 #define CK(...)                        \
   do {                                 \
@@ -699,7 +747,15 @@ extern "C" int remd_gpu_create(remd_gpu **out, const remd_gpu_desc *d, const rem
       HIPCHK(hipHostMalloc(&g->h_abort, sizeof(unsigned), hipHostMallocDefault));
       *g->h_abort = 0u;
     }
-    if (g->grec) HIPCHK(hipMalloc(&g->d_grec, R * rec_bytes((int)N, g->NS, g->prm.precision)));
+    if (!g->resident && g->gparts > 1) {
+      HIPCHK(hipMalloc(&g->d_sync, sizeof(unsigned long long) * (R + 1)));
+      HIPCHK(hipMemsetAsync(g->d_sync, 0, sizeof(unsigned long long) * (R + 1), g->stream));
+      HIPCHK(hipMalloc(&g->d_xbuf, sizeof(double) * R * grow_doubles((int)N)));
+      HIPCHK(hipMalloc(&g->d_gbuf, sizeof(double) * R * g->gparts * gm_part_doubles((int)N)));
+      HIPCHK(hipHostMalloc(&g->h_abort, sizeof(unsigned), hipHostMallocDefault));
+      *g->h_abort = 0u;
+    }
+    if (g->grec) HIPCHK(hipMalloc(&g->d_grec, R * g->gparts * rec_bytes((int)N, g->NS, g->prm.precision)));
     return 0;
   }());
   CK(build_wall(g));
@@ -915,10 +971,11 @@ extern "C" int remd_gpu_execute_steps_plain(remd_gpu *g, const double *T, const 
     a.abort = g->d_sync ? (unsigned *)(g->d_sync + g->nrep) : nullptr;
     if (g->resident) {
       rc = launch_res(g, a, g->stream);
-      if (rc) return rc;
     } else {
-      HIPCHK(launch_interval(a, g->nt, g->NS, g->prm.precision, g->lds, g->stream));
+      rc = launch_global(g, a, g->stream);
+      g->last_parts = a.parts;
     }
+    if (rc) return rc;
   }
   HIPCHK(hipEventRecord(g->ev1, g->stream));
   if (parts > 1)
@@ -1526,14 +1583,15 @@ extern "C" int remd_gpu_execute_intervals(remd_gpu *g, int ntemp, int npress, lo
     HIPCHK(hipEventRecord(g->xi_ev[2 * k], g->stream));
     if (g->resident) {
       rc = launch_res(g, a, g->stream);
-      if (rc) return rc;
     } else {
-      HIPCHK(launch_interval(a, g->nt, g->NS, g->prm.precision, g->lds, g->stream));
+      rc = launch_global(g, a, g->stream);
+      g->last_parts = a.parts;
     }
+    if (rc) return rc;
     HIPCHK(hipEventRecord(g->xi_ev[2 * k + 1], g->stream));
     HIPCHK(launch_exchange(g->xi_jobs + k, 1, g->stream));
   }
-  if (a.parts > 1)
+  if (g->resident && a.parts > 1)
     HIPCHK(hipMemcpyAsync(g->h_abort, a.abort, sizeof(unsigned), hipMemcpyDeviceToHost, g->stream));
   std::vector<int> acc(U > 0 ? U : 1);
   std::vector<double> hist(averages ? (size_t)NSC * R * nint : 0);

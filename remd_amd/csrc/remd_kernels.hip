@@ -195,6 +195,7 @@ struct Lds {
   uint16_t *js, *je;
   double *red;   // NW x 32 doubles
   int *cnt;      // radix counts
+  int *flag;     // group barrier status (the counts' area, idle outside the sort)
   MaskBuf mask;  // what the launch's LDS leaves
 };
 
@@ -212,6 +213,7 @@ __device__ inline Lds lds_carve(char *smem, int nmol, int nsite, int prec, int l
   char *misc = smem + region0 + align16(4 * nmol);
   L.red = (double *)misc;
   L.cnt = (int *)(misc + (NT / WAVE) * 32 * 8);
+  L.flag = L.cnt;
   const int base = lds_bytes(nmol, nsite, prec, NT, grec != nullptr);
   L.mask.buf = (unsigned *)(smem + base);
   L.mask.words = lds > base ? (lds - base) / (8 * NT) * 2 : 0;
@@ -1244,10 +1246,99 @@ __device__ void m2a(JRef J, const double *mol, int N, double L0, double L1, doub
   }
 }
 
-// Pair pass + wall + A2M for every molecule of the replica.  Writes f, n
-// into the molecule block and the energy/virial totals into c.
+// ------------------------------------------------- workgroups of a replica
+constexpr unsigned MAXSPIN = 1u << 20; // group-barrier polls before the launch gives up
+
+struct Group {
+  int parts, part;
+  unsigned long long *ctr;  // low 32 bits: arrivals of this replica's parts; zero at start
+  unsigned *abort;  // nonzero once any wait of the launch timed out
+  double *xbuf;     // 2 x xbuf_parity_doubles(N) exchange rows (double-buffered by step parity)
+  unsigned epoch;   // group barriers completed in this launch
+  bool same_xcd;    // every part of the replica shares one L2
+  int mode;         // same-XCD barrier variant (LaunchArgs::same_xcd_mode)
+};
+
+// XCD (XCC) this workgroup runs on.
+__device__ inline unsigned xcc_id() { return __builtin_amdgcn_s_getreg((3 << 11) | (0 << 6) | 20) & 15u; }
+
+// Barrier across the parts of one replica.  Every thread first makes its
+// own global stores visible to the other parts; one thread counts in and
+// polls the counter (bounded; a timeout raises the launch-wide abort flag so
+// every part leaves); then the other parts' stores are made visible to this
+// part's loads.  When all parts share one XCD (and so one L2, the coherence
+// point of its CUs) the stores are only drained to L2 and the exchange rows
+// are read with device-scope loads that bypass the CU's L1 (an L1-only
+// invalidate was measured not to suffice); otherwise agent-scope release and
+// acquire fences (L2 write-back / invalidate) and ordinary loads.  Returns
+// false when the launch is aborting.
+// `census` (the launch's first barrier, fully fenced): each part also leaves
+// its XCD in its slot at the start of the exchange area -- the rows of even
+// epochs, written again only after every part has passed the next barrier --
+// and flag[1] receives whether all parts share one XCD; every part reads the
+// same slots, so all decide alike.
+template <int NT>
+__device__ bool group_wait(Group &g, int *flag, double *pt_sc = nullptr, bool census = false) {
+  PT_DECL
+  (void)pt_sc;
+  unsigned *slots = (unsigned *)g.xbuf;
+  if (census && threadIdx.x == 0)
+    __hip_atomic_store(slots + g.part, xcc_id(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (g.same_xcd && !(g.mode & 1)) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  else __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+  __syncthreads();
+  PT_MARK(8, pt_sc);
+  if (threadIdx.x == 0) {
+    int ok = 1;
+    const unsigned long long target = (unsigned long long)g.parts * (g.epoch + 1u);
+    __hip_atomic_fetch_add(g.ctr, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    unsigned spins = 0;
+    while ((__hip_atomic_load(g.ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & 0xffffffffull) < target) {
+      ++spins;
+      if ((spins & 63u) == 0u) {
+        if (__hip_atomic_load(g.abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) {
+          ok = 0;
+          break;
+        }
+        if (spins > MAXSPIN) {
+          __hip_atomic_store(g.abort, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          ok = 0;
+          break;
+        }
+      }
+      __builtin_amdgcn_s_sleep(2);
+    }
+    *flag = ok;
+    if (census) {
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+      int same = 1;
+      for (int p = 0; ok && p < g.parts; p++)
+        same &= __hip_atomic_load(slots + p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == xcc_id() ? 1 : 0;
+      flag[1] = same;
+    }
+  }
+  __syncthreads();
+  PT_MARK(9, pt_sc);
+  const bool ok = *flag != 0;
+  if (!g.same_xcd || (g.mode & 2)) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  g.epoch++;
+  // no barrier needed before flag is rewritten: thread 0 writes it again
+  // only after the workgroup barrier that opens the next call, which every
+  // thread reaches after its read above
+  PT_MARK(10, pt_sc);
+  return ok;
+}
+
+// Pair pass + wall + A2M for the molecules of this part (all of them when
+// the replica has one workgroup).  Writes f, n into the molecule block and
+// the energy/virial totals into c.  A replica split over parts exchanges one
+// row per molecule (F, n, lj, clmb, wall, virial) and every part adds the
+// energies in the order of the one-workgroup form -- thread t adds the
+// molecules whose first chunk falls on it, in order, then the workgroup tree
+// -- so the bits do not depend on the parts.  Returns false when the launch
+// is aborting.
 template <int NT, int NS, typename PT>
-__device__ void force_pass(JRef J, double *mol, int N, Sc &c, const Lds &S,
+__device__ bool force_pass(JRef J, double *mol, int N, Sc &c, const Lds &S, Group &g,
                            double *site_dbg, double *pt_sc) {
   PT_DECL
   constexpr int QB = (NS == 3) ? 0 : 1;
@@ -1302,11 +1393,15 @@ __device__ void force_pass(JRef J, double *mol, int N, Sc &c, const Lds &S,
   const double dr = (J.cmode == 1) ? J.wall_length / (double)J.nfwall
                                    : 0.5 * J.wall_length / (double)J.nfwall;
   const double dri = 1.0 / dr;
-  const int total = N << lc;
+  const bool split = g.parts > 1;
+  const int i0 = split ? (int)(((long long)g.part * N) / g.parts) : 0;
+  const int i1 = split ? (int)(((long long)(g.part + 1) * N) / g.parts) : N;
+  double *row = split ? g.xbuf + (size_t)(g.epoch & 1u) * GR * N : nullptr;
+  const int total = (i1 - i0) << lc;
   for (int base = 0; base < total; base += NT) {
     const int t = base + threadIdx.x;
     const bool active = t < total;
-    const int i = active ? (t >> lc) : 0;
+    const int i = i0 + (active ? (t >> lc) : 0);
     const int cc = t & (C - 1);
     Acc<NS> acc;
 #pragma unroll
@@ -1352,6 +1447,7 @@ __device__ void force_pass(JRef J, double *mol, int N, Sc &c, const Lds &S,
         for (int a = 0; a < NS; a++) s += acc.site[a][d];
         F[d] = s;
       }
+      double ew = 0.0;
       if (J.cmode == 1 || J.cmode == 2) {
         double b0[3];
         body_to_space(q, (const double *)J.site_r[0], b0);
@@ -1367,7 +1463,7 @@ __device__ void force_pass(JRef J, double *mol, int N, Sc &c, const Lds &S,
           acc.site[0][1] += f * y;
           F[0] += f * x;
           F[1] += f * y;
-          e_wall += e;
+          ew = e;
         } else {
           const double z = (mol[F_RZ * N + i] - 0.5) * c.L[2] + b0[2];
           const double az = fabs(z);
@@ -1377,7 +1473,7 @@ __device__ void force_pass(JRef J, double *mol, int N, Sc &c, const Lds &S,
           const double e = (J.fwall[2 * (idx + 1) + 1] - J.fwall[2 * idx + 1]) * dri * (az - dr * idx) + J.fwall[2 * idx + 1];
           acc.site[0][2] += f * z;
           F[2] += f * z;
-          e_wall += e;
+          ew = e;
         }
       }
       // A2M torque (src/molecules.cxx:409-418)
@@ -1405,12 +1501,53 @@ __device__ void force_pass(JRef J, double *mol, int N, Sc &c, const Lds &S,
 #pragma unroll
           for (int d = 0; d < 3; d++) site_dbg[(i * NS + a) * 3 + d] = acc.site[a][d];
       }
-      e_lj += acc.lj;
-      e_cl += acc.clmb;
-      vir[0] += acc.vir[0];
-      vir[1] += acc.vir[1];
-      vir[2] += acc.vir[2];
+      if (split) {
+        const double v[GR] = {F[0],       F[1],       F[2],       n4[0],  n4[1],    n4[2], n4[3],
+                              acc.vir[0], acc.vir[1], acc.vir[2], acc.lj, acc.clmb, ew};
+#pragma unroll
+        for (int u = 0; u < GR; u++) row[(size_t)u * N + i] = v[u];
+      } else {
+        e_lj += acc.lj;
+        e_cl += acc.clmb;
+        e_wall += ew;
+        vir[0] += acc.vir[0];
+        vir[1] += acc.vir[1];
+        vir[2] += acc.vir[2];
+      }
     }
+  }
+  if (split) {
+    if (!group_wait<NT>(g, S.flag, pt_sc)) return false;
+    const bool direct = g.same_xcd && !(g.mode & 2);
+    auto get = [&](int u, int i) {
+      const double *o = row + (size_t)u * N + i;
+      return direct ? __hip_atomic_load(o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : *o;
+    };
+    // the other parts' forces and torques
+    for (int i = threadIdx.x; i < N; i += NT) {
+      if (i >= i0 && i < i1) continue;
+      double v[7];
+#pragma unroll
+      for (int u = 0; u < 7; u++) v[u] = get(u, i);
+#pragma unroll
+      for (int u = 0; u < 3; u++) mol[(F_FX + u) * N + i] = v[u];
+#pragma unroll
+      for (int u = 0; u < 4; u++) mol[(F_N0 + u) * N + i] = v[3 + u];
+    }
+    // energies and virial, in the order of the one-workgroup form
+    const int t = threadIdx.x;
+    if ((t & (C - 1)) == 0)
+      for (int i = t >> lc; i < N; i += NT >> lc) {
+        double v[6];
+#pragma unroll
+        for (int u = 0; u < 6; u++) v[u] = get(7 + u, i);
+        vir[0] += v[0];
+        vir[1] += v[1];
+        vir[2] += v[2];
+        e_lj += v[3];
+        e_cl += v[4];
+        e_wall += v[5];
+      }
   }
   PT_MARK(5, pt_sc);
   double tot[6] = {e_lj, e_cl, e_wall, vir[0], vir[1], vir[2]};
@@ -1423,6 +1560,7 @@ __device__ void force_pass(JRef J, double *mol, int N, Sc &c, const Lds &S,
   c.vir[1] = 0.5 * tot[4];
   c.vir[2] = 0.5 * tot[5];
   c.pot = c.lj + c.clmb + c.wall;
+  return true;
 }
 
 // ----------------------------------------------------------- one step
@@ -1548,45 +1686,72 @@ __device__ void second_half(JRef J, double *mol, int N, Sc &c) {
   __syncthreads();
 }
 
+// One step.  With `fuse` the second half of the previous step runs inside
+// the first half's molecule loop; `last` adds this step's own second half.
 template <int NT, int NS, typename PT>
-__device__ void md_step(JRef J, double *mol, int *mid, int N, Sc &c, const Lds &S,
-                        bool do_sort, const DescD &R) {
+__device__ bool md_step(JRef J, double *mol, int *mid, int N, Sc &c, const Lds &S, Group &g, bool fuse, bool last,
+                        bool do_sort, double *site_dbg, int *win_dbg, double *pt_sc) {
   PT_DECL
-  first_half<NT>(J, mol, N, c, S.red);
-  PT_MARK(0, gen(R.sc) + S_DIAG0);
+  if (fuse) first_half<NT, true>(J, mol, N, c, S.red);
+  else first_half<NT, false>(J, mol, N, c, S.red);
+  PT_MARK(0, pt_sc);
   // force
-  if (do_sort) sort_and_window<NT>(J, mol, mid, N, J.sort_axis == 0 ? c.L[0] : c.L[2], J.margin, S, gen(R.win));
-  PT_MARK(1, gen(R.sc) + S_DIAG0);
-  force_pass<NT, NS, PT>(J, mol, N, c, S, gen(R.site_f), gen(R.sc) + S_DIAG0);  // ends with block_sum (synced)
-  PT_MARK(2, gen(R.sc) + S_DIAG0);
-  second_half<NT>(J, mol, N, c);
-  PT_MARK(3, gen(R.sc) + S_DIAG0);
+  if (do_sort) sort_and_window<NT>(J, mol, mid, N, J.sort_axis == 0 ? c.L[0] : c.L[2], J.margin, S, win_dbg);
+  PT_MARK(1, pt_sc);
+  if (!force_pass<NT, NS, PT>(J, mol, N, c, S, g, site_dbg, pt_sc)) return false;  // ends with block_sum (synced)
+  PT_MARK(2, pt_sc);
+  if (last) second_half<NT>(J, mol, N, c);
+  PT_MARK(3, pt_sc);
+  return true;
 }
 
 // --------------------------------------------------------- replica driver
+// A replica may be split over parts (workgroups of one XCD, as on the
+// resident path): each part then keeps a private copy of the state in
+// R.gbuf (and of the site records in R.grec, where they do not fit the LDS),
+// integrates all of it and evaluates the forces of its own molecules; the
+// lead part writes the state back.  One workgroup works on the state itself.
 template <int NT, int NS, typename PT>
-__device__ void run_replica(const LaunchArgs &a, const DescD &R, JRef J, char *smem) {
+__device__ void run_replica(const LaunchArgs &a, const DescD &R, JRef J, Group &g, char *smem) {
   const int N = J.nmol;
+  const bool split = g.parts > 1;
+  const bool lead = g.part == 0;
   double *mol = gen(R.mol);
   int *mid = gen(R.mid);
-  Lds S = lds_carve<NT>(smem, N, NS, J.precision, a.lds, gen(R.grec));
+  char *grec = gen(R.grec);
+  if (split && grec) grec += (size_t)g.part * rec_bytes(N, NS, J.precision);
+  Lds S = lds_carve<NT>(smem, N, NS, J.precision, a.lds, grec);
   Sc c;
   load_sc(c, gen(R.sc));
+  const double xflag = gen(R.sc)[S_XFLAG];
+  const double Tn = gen(R.sc)[S_TNEW];
+  const double Pn = gen(R.sc)[S_PNEW];
+  if (split) {
+    mol = gen(R.gbuf) + (size_t)g.part * gm_part_doubles(N);
+    mid = (int *)(mol + (size_t)NFIELD * N);
+    for (int k = threadIdx.x; k < NFIELD * N; k += NT) mol[k] = gen(R.mol)[k];
+    for (int i = threadIdx.x; i < N; i += NT) mid[i] = gen(R.mid)[i];
+    g.same_xcd = false;
+    if (!group_wait<NT>(g, S.flag, nullptr, true)) return;
+    g.same_xcd = a.same_xcd_ok && S.flag[1] != 0;
+    __syncthreads();
+  }
+  double *sc_out = lead ? gen(R.sc) : nullptr;
+  int *win = lead ? gen(R.win) : nullptr;
+  double *site_dbg = gen(R.site_f);
+  double *pt = lead ? gen(R.sc) + S_DIAG0 : nullptr;
 
   if (a.mode == MODE_INIT) {
     // InitializeProperty (src/molecules.h:260-270): sort with margin 0,
     // force, gkT, CalcProperties, H0 = tot.
-    sort_and_window<NT>(J, mol, mid, N, J.sort_axis == 0 ? c.L[0] : c.L[2], 0.0, S, gen(R.win));
-    force_pass<NT, NS, PT>(J, mol, N, c, S, gen(R.site_f), gen(R.sc) + S_DIAG0);
+    sort_and_window<NT>(J, mol, mid, N, J.sort_axis == 0 ? c.L[0] : c.L[2], 0.0, S, win);
+    if (!force_pass<NT, NS, PT>(J, mol, N, c, S, g, site_dbg, pt)) return;
     c.gkT = 6.0 * (double)N * c.T;
     const double tot = total_energy<NT>(J, mol, N, c, S.red);
     c.H0 = tot;
-    calc_properties<NT>(J, mol, N, c, gen(R.sc), S.red);
-    if (threadIdx.x == 0) store_sc(c, gen(R.sc));
-    return;
-  }
-  if (a.mode == MODE_FORCE) {
-    if (a.do_sort) sort_and_window<NT>(J, mol, mid, N, J.sort_axis == 0 ? c.L[0] : c.L[2], a.margin, S, gen(R.win));
+    calc_properties<NT>(J, mol, N, c, sc_out, S.red);
+  } else if (a.mode == MODE_FORCE) {
+    if (a.do_sort) sort_and_window<NT>(J, mol, mid, N, J.sort_axis == 0 ? c.L[0] : c.L[2], a.margin, S, win);
     else {
       // reuse the stored window
       for (int i = threadIdx.x; i < N; i += NT) {
@@ -1603,59 +1768,86 @@ __device__ void run_replica(const LaunchArgs &a, const DescD &R, JRef J, char *s
       }
       __syncthreads();
     }
-    force_pass<NT, NS, PT>(J, mol, N, c, S, gen(R.site_f), gen(R.sc) + S_DIAG0);
-    calc_properties<NT>(J, mol, N, c, gen(R.sc), S.red);
-    if (threadIdx.x == 0) store_sc(c, gen(R.sc));
-    return;
-  }
-
-  // MODE_INTERVAL
-  const double xflag = gen(R.sc)[S_XFLAG];
-  if (xflag != 0.0) {
-    // REMD::ReplicaExchange for an exchanged replica
-    // (src/remd.cxx:526-536): ChangeTemperature, KillMomentum, SetPressure,
-    // CalcProperties, UpdateHamiltonian.
-    const double Tn = gen(R.sc)[S_TNEW];
-    const double coef = sqrt(Tn / c.T);
-    for (int i = threadIdx.x; i < N; i += NT) {
-      for (int d = 0; d < 3; d++) mol[(F_VX + d) * N + i] *= coef / c.s;
-      for (int d = 0; d < 4; d++) mol[(F_P0 + d) * N + i] *= coef / c.s;
+    if (!force_pass<NT, NS, PT>(J, mol, N, c, S, g, site_dbg, pt)) return;
+    calc_properties<NT>(J, mol, N, c, sc_out, S.red);
+  } else {
+    // MODE_INTERVAL
+    if (xflag != 0.0) {
+      // REMD::ReplicaExchange for an exchanged replica
+      // (src/remd.cxx:526-536): ChangeTemperature, KillMomentum, SetPressure,
+      // CalcProperties, UpdateHamiltonian.
+      const double coef = sqrt(Tn / c.T);
+      for (int i = threadIdx.x; i < N; i += NT) {
+        for (int d = 0; d < 3; d++) mol[(F_VX + d) * N + i] *= coef / c.s;
+        for (int d = 0; d < 4; d++) mol[(F_P0 + d) * N + i] *= coef / c.s;
+      }
+      c.Ps *= coef;
+      if (J.pmode == 1) c.Pv[0] *= coef * c.s;
+      if (J.pmode == 2) c.Pv[2] *= coef * c.s;
+      if (J.pmode == 3) c.Pv[0] *= coef * c.s;
+      c.T = Tn;
+      c.gkT = 6.0 * (double)N * Tn;
+      c.s = 1.0;
+      __syncthreads();
+      kill_momentum<NT>(J, mol, N, c, S.red, false);
+      c.P = Pn;
+      c.H0 = total_energy<NT>(J, mol, N, c, S.red);
     }
-    c.Ps *= coef;
-    if (J.pmode == 1) c.Pv[0] *= coef * c.s;
-    if (J.pmode == 2) c.Pv[2] *= coef * c.s;
-    if (J.pmode == 3) c.Pv[0] *= coef * c.s;
-    c.T = Tn;
-    c.gkT = 6.0 * (double)N * Tn;
-    c.s = 1.0;
-    __syncthreads();
-    kill_momentum<NT>(J, mol, N, c, S.red, false);
-    c.P = gen(R.sc)[S_PNEW];
-    c.H0 = total_energy<NT>(J, mol, N, c, S.red);
-  }
-  // the driver scales once per interval before ExecuteSteps
-  // (src/remd.cxx:259-262), which scales again at every step
-  if (J.tmode == 2) velocity_scaling<NT>(J, mol, N, c, S.red);
-  for (int st = 0; st < J.interval; ++st) {
+    // the driver scales once per interval before ExecuteSteps
+    // (src/remd.cxx:259-262), which scales again at every step
     if (J.tmode == 2) velocity_scaling<NT>(J, mol, N, c, S.red);
-    const bool do_sort = (st % J.sort_interval) == 0;
-    md_step<NT, NS, PT>(J, mol, mid, N, c, S, do_sort, R);
+    const bool fuse = J.tmode != 2;
+    for (int st = 0; st < J.interval; ++st) {
+      if (J.tmode == 2) velocity_scaling<NT>(J, mol, N, c, S.red);
+      if (!md_step<NT, NS, PT>(J, mol, mid, N, c, S, g, fuse && st > 0, !fuse || st == J.interval - 1,
+                               (st % J.sort_interval) == 0, site_dbg, win, pt))
+        return;
+    }
+    calc_properties<NT>(J, mol, N, c, sc_out, S.red);
   }
-  calc_properties<NT>(J, mol, N, c, gen(R.sc), S.red);
-  if (threadIdx.x == 0) {
+  if (split) {
+    // every part has read the state (the first barrier); the lead writes it
+    if (lead) {
+      for (int k = threadIdx.x; k < NFIELD * N; k += NT) gen(R.mol)[k] = mol[k];
+      for (int i = threadIdx.x; i < N; i += NT) gen(R.mid)[i] = mid[i];
+    }
+  }
+  if (lead && threadIdx.x == 0) {
     store_sc(c, gen(R.sc));
-    gen(R.sc)[S_XFLAG] = 0.0;
-    gen(R.sc)[S_STEPS] += (double)J.interval;
+    if (a.mode == MODE_INTERVAL) {
+      gen(R.sc)[S_XFLAG] = 0.0;
+      gen(R.sc)[S_STEPS] += (double)J.interval;
+    }
+    if (split) __hip_atomic_fetch_or(g.ctr, REPLICA_DONE, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 
+// grid: as resident_kernel's (parts of a replica on block indices equal mod
+// 8).  a.skip_done: the replicas that finished in an aborted launch of the
+// same interval (REPLICA_DONE in their group word) are left alone.
 template <int NT, int NS, typename PT>
 __global__ __launch_bounds__(NT) void interval_kernel(LaunchArgs a) {
   extern __shared__ __align__(16) char smem[];
-  if ((int)blockIdx.x >= a.nrep) return;
-  const DescD R = ((const DescD *)a.reps)[blockIdx.x];
+  int rep = blockIdx.x, part = 0;
+  if (a.parts > 1) {
+    const int slot = rep >> 3;
+    rep = (slot / a.parts) * 8 + (rep & 7);
+    part = slot % a.parts;
+  }
+  if (rep >= a.nrep) return;
+  if (a.skip_done && (a.sync[rep] & REPLICA_DONE)) return;
+  const DescD R = ((const DescD *)a.reps)[rep];
   JRef J = *R.job;
-  run_replica<NT, NS, PT>(a, R, J, smem);
+  Group g;
+  g.parts = a.parts < 1 ? 1 : a.parts;
+  g.part = part;
+  g.ctr = a.sync ? a.sync + rep : nullptr;
+  g.abort = a.abort;
+  g.xbuf = gen(R.xbuf);
+  g.epoch = 0;
+  g.same_xcd = false;
+  g.mode = a.same_xcd_mode;
+  run_replica<NT, NS, PT>(a, R, J, g, smem);
 }
 
 // ====================================================== replica-resident path
@@ -1669,8 +1861,6 @@ __global__ __launch_bounds__(NT) void interval_kernel(LaunchArgs a) {
 // is computed whole by one part with the job's fixed chunk count, and the
 // energies are reduced from per-molecule values in a fixed order, so results
 // do not depend on G, on batching or on placement.
-
-constexpr unsigned MAXSPIN = 1u << 20; // group-barrier polls before the launch gives up
 
 // Per-item partials of the pair pass: COM force (3), quaternion torque (4),
 // virial (3), lj, clmb, wall energy -- plus the site forces (3 NS) when the
@@ -1741,86 +1931,6 @@ __device__ inline LdsR carve_resident(char *smem, int N, int prec, bool site_dbg
   p += 64;
   L.ptimer = (double *)p;
   return L;
-}
-
-struct Group {
-  int parts, part;
-  unsigned long long *ctr;  // low 32 bits: arrivals of this replica's parts; high 32 bits: 4-bit
-                            // count of parts per XCD (added at the first barrier); zero at start
-  unsigned *abort;  // nonzero once any wait of the launch timed out
-  double *xbuf;     // 2 x xbuf_parity_doubles(N) exchange rows (double-buffered by step parity)
-  unsigned epoch;   // group barriers completed in this launch
-  bool same_xcd;    // every part of the replica shares one L2
-  int mode;         // same-XCD barrier variant (LaunchArgs::same_xcd_mode)
-};
-
-// XCD (XCC) this workgroup runs on.
-__device__ inline unsigned xcc_id() { return __builtin_amdgcn_s_getreg((3 << 11) | (0 << 6) | 20) & 15u; }
-
-// Barrier across the parts of one replica.  Every thread first makes its
-// own global stores visible to the other parts; one thread counts in and
-// polls the counter (bounded; a timeout raises the launch-wide abort flag so
-// every part leaves); then the other parts' stores are made visible to this
-// part's loads.  When all parts share one XCD (and so one L2, the coherence
-// point of its CUs) the stores are only drained to L2 and the exchange rows
-// are read with device-scope loads that bypass the CU's L1 (an L1-only
-// invalidate was measured not to suffice); otherwise agent-scope release and
-// acquire fences (L2 write-back / invalidate) and ordinary loads.  Returns
-// false when the launch is aborting.
-// `census` (the launch's first barrier): each part also adds 1 to the
-// 4-bit field of its XCD in the high half of the group word, and flag[1]
-// receives whether all parts share one XCD -- read from the same word that
-// completes the barrier, so every part sees every part's field and all
-// parts decide alike.
-template <int NT>
-__device__ bool group_wait(Group &g, int *flag, double *pt_sc = nullptr, bool census = false) {
-  PT_DECL
-  (void)pt_sc;
-  if (g.same_xcd && !(g.mode & 1)) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  else __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-  __syncthreads();
-  PT_MARK(8, pt_sc);
-  if (threadIdx.x == 0) {
-    int ok = 1;
-    const unsigned long long target = (unsigned long long)g.parts * (g.epoch + 1u);
-    const unsigned long long inc = 1ull + (census ? (1ull << (32 + 4 * xcc_id())) : 0ull);
-    __hip_atomic_fetch_add(g.ctr, inc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    unsigned spins = 0;
-    unsigned long long v;
-    while (((v = __hip_atomic_load(g.ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) & 0xffffffffull) <
-           target) {
-      ++spins;
-      if ((spins & 63u) == 0u) {
-        if (__hip_atomic_load(g.abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) {
-          ok = 0;
-          break;
-        }
-        if (spins > MAXSPIN) {
-          __hip_atomic_store(g.abort, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          ok = 0;
-          break;
-        }
-      }
-      __builtin_amdgcn_s_sleep(2);
-    }
-    *flag = ok;
-    if (census) {
-      const unsigned hist = (unsigned)(v >> 32);
-      int nz = 0;
-      for (int x = 0; x < 8; x++) nz += ((hist >> (4 * x)) & 15u) != 0u;
-      flag[1] = (nz == 1) ? 1 : 0;
-    }
-  }
-  __syncthreads();
-  PT_MARK(9, pt_sc);
-  const bool ok = *flag != 0;
-  if (!g.same_xcd || (g.mode & 2)) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-  g.epoch++;
-  // no barrier needed before flag is rewritten: thread 0 writes it again
-  // only after the workgroup barrier that opens the next call, which every
-  // thread reaches after its read above
-  PT_MARK(10, pt_sc);
-  return ok;
 }
 
 // Sorted position rk[i] of each key ax[i] (stable: equal keys keep their
@@ -2960,7 +3070,7 @@ hipError_t launch_interval(const LaunchArgs &a, int nt, int nsite, int prec, int
   if (a.nrep <= 0) return hipSuccess;
   LaunchArgs arg = a;
   arg.lds = lds;
-  return launch_fn(interval_fn(nt, nsite, prec), a.nrep, nt, arg, lds, st);
+  return launch_fn(interval_fn(nt, nsite, prec), resident_grid(a.nrep, a.parts), nt, arg, lds, st);
 }
 
 hipError_t set_kernel_lds_limit(int bytes) {

@@ -9,6 +9,22 @@ import remd_amd as ra
 pytestmark = pytest.mark.gpu
 
 
+def _bulk(nmol, model, nrep=2, seed=17):
+    from remd_amd import inputs
+
+    L = max((nmol * 29.9) ** (1.0 / 3.0), 19.2)
+    s = inputs.config_bulk(seed=seed, nmol=nmol, L=L, ntemp=nrep, npress=1, model=model) if nmol <= 343 else None
+    if s is None:
+        s = inputs.config_bulk(seed=seed, nmol=343, L=L, ntemp=nrep, npress=1, model=model)
+        rng = np.random.RandomState(seed)
+        s.nmol = nmol
+        s.states = inputs._states(rng, inputs.molecule(model), inputs.place_lattice(nmol, L), s.T, (L, L, L), 0.5, 0.05)
+    s.pconstant = 1
+    s.dt_fs = 0.2  # unrelaxed contacts
+    s.interval = 12  # two sorts
+    return s
+
+
 @pytest.mark.parametrize("nfw", [3, 4, 5, 7, 1003])
 def test_wall_table_tube_node_counts(nfw):
     """Tables whose node count is below, at and beside the nodes of one
@@ -34,15 +50,7 @@ def test_screened_pairs_match_oracle(model, nmol, chunks, path, precision):
     force is a sum of about 100 pairs rounded at 6e-8 each, against terms up
     to 50 times the sum); FP64: 1e-11."""
     from helpers import oracle_for, rel_rms
-    from remd_amd import inputs
-
-    L = max((nmol * 29.9) ** (1.0 / 3.0), 19.2)
-    s = inputs.config_bulk(seed=11, nmol=nmol, L=L, ntemp=1, npress=1, model=model) if nmol <= 343 else None
-    if s is None:
-        s = inputs.config_bulk(seed=11, nmol=343, L=L, ntemp=1, npress=1, model=model)
-        rng = np.random.RandomState(11)
-        s.nmol = nmol
-        s.states = inputs._states(rng, inputs.molecule(model), inputs.place_lattice(nmol, L), s.T, (L, L, L), 0.5, 0.05)
+    s = _bulk(nmol, model, nrep=1, seed=11)
     o = oracle_for(s)
     o.initialize_property()
     g = ra.REMDGPU(s, precision=precision, chunks=chunks, path=path)
@@ -62,3 +70,34 @@ def test_tube_screening_rule(R):
     o.initialize_property()
     g = ra.REMDGPU(s)
     assert rel_rms(g.state(0)["f"], o.state()["f"]) < 1e-5
+
+
+@pytest.mark.parametrize("model,nmol,chunks,precision,abort", [
+    ("TIP4P", 513, 1, 0, False),   # ragged parts
+    ("TIP3P", 600, 4, 0, False),   # butterfly over chunks
+    ("TIP5P", 700, 2, 1, False),   # FP64
+    ("TIP4P", 2100, 1, 1, False),  # site records in global memory, one copy per part
+    ("TIP4P", 600, 1, 0, True),    # parts that give up: completed by one workgroup per replica
+])
+def test_global_path_parts_keep_the_bits(model, nmol, chunks, precision, abort, monkeypatch):
+    """A global-state job alone is split over workgroups, in a batch it is
+    not: the same bits, also when the split launch gives up."""
+    s = _bulk(nmol, model)
+    a = ra.REMDGPU(s, precision=precision, chunks=chunks, path=ra.PATH_GLOBAL)
+    b = ra.REMDGPU(s, precision=precision, chunks=chunks, path=ra.PATH_GLOBAL)
+    if abort:
+        monkeypatch.setenv("REMD_GLOBAL_ABORT", "1")
+    a.execute_steps(s.T, s.P)
+    monkeypatch.delenv("REMD_GLOBAL_ABORT", raising=False)
+    if not abort:
+        assert a.launch_path()[1] > 1
+    bt = ra.Batch()
+    bt.add(b)
+    b.set_conditions(s.T, s.P)
+    bt.execute()
+    assert np.array_equal(a.all_averages(), b.all_averages())
+    for r in range(s.nreplica):
+        x, y = a.state(r), b.state(r)
+        for k in ("r", "v", "f", "q", "p", "n", "id", "scal"):
+            assert np.array_equal(x[k], y[k]), k
+    bt.close()
