@@ -1039,17 +1039,6 @@ __device__ __forceinline__ void load_com(PT (&c)[3], const PT *rec, int N, int j
   else c[2] = rec_vec<VW, PT>(rec, N, 1, j).v[0];
 }
 
-// |COM difference| on axis d reduced to the nearest image, for screening
-// only (the sign is lost and the rounding is not min_image's): both
-// coordinates lie in the box, so |x| < L; on the non-periodic axes L = 0 and
-// the minimum is -|x|.
-template <int PER, int NS, typename PT>
-__device__ __forceinline__ PT near_image(PT x, const PairK<NS, PT> &k, int d) {
-  const PT a = fabs(x);
-  if constexpr (PER < 0) return fmin(a, k.L[d] - a);
-  else return ((PER >> d) & 1) ? fmin(a, k.L[d] - a) : x;
-}
-
 // Screening of `n` <= 32 partners jj, jj + C, ... of a work item by COM
 // distance, radius slightly above the cutoff (pair_acc decides): bit u of
 // the result is partner u; molecule i itself passes.  The COMs are loaded
@@ -1074,7 +1063,7 @@ __device__ __forceinline__ unsigned screen(const PT *rec, int N, int jj, int C, 
     for (int u = 0; u < SCREEN_BATCH; u++) {
       PT dg[3];
 #pragma unroll
-      for (int d = 0; d < 3; d++) dg[d] = near_image<PER>(gi[d] - c[u][d], k, d);
+      for (int d = 0; d < 3; d++) dg[d] = min_image<PER>(gi[d] - c[u][d], k, d);
       const PT r2 = dg[0] * dg[0] + dg[1] * dg[1] + dg[2] * dg[2];
       m |= (r2 < k.rs2 ? 1u : 0u) << u;
     }
@@ -1098,8 +1087,10 @@ __device__ __forceinline__ unsigned screen(const PT *rec, int N, int jj, int C, 
 // the pair loop is then at the FP32 issue rate of its one wave per SIMD.
 // Both loops are wave-uniform: a lane past its last partner takes the
 // molecule itself, which adds nothing.
+// Returns whether the item has partners: where it has none the caller drops
+// the sums (self-evaluations of a state gone non-finite are not zeros).
 template <int NT, int NS, int QB, typename PT, int PER, bool RECORDS, typename AT>
-__device__ __forceinline__ void pair_window_run(const PT *rec, int N, int i, int js, int je, int c0, int C,
+__device__ __forceinline__ bool pair_window_run(const PT *rec, int N, int i, int js, int je, int c0, int C,
                                                 bool compact, const PT *gi, const PT (&ai)[NS][3],
                                                 const PairK<NS, PT> &k, const MaskBuf &mb, Acc<NS, AT> &acc) {
   constexpr int RL = 3 + 3 * NS;
@@ -1116,7 +1107,8 @@ __device__ __forceinline__ void pair_window_run(const PT *rec, int N, int i, int
     };
     PT ra[RL], rb[RL];
     int ja, jb;
-    if (!fetch(ra, ja)) return;
+    const bool some = jj <= je;
+    if (!fetch(ra, ja)) return false;
     for (;;) {
       const bool more_b = fetch(rb, jb);
       pair_acc<NS, QB, PT, PER>(gi, ai, ra, k, ja == i, acc);
@@ -1125,8 +1117,9 @@ __device__ __forceinline__ void pair_window_run(const PT *rec, int N, int i, int
       pair_acc<NS, QB, PT, PER>(gi, ai, rb, k, jb == i, acc);
       if (!more_a) break;
     }
-    return;
+    return some;
   }
+  bool some = false;
   int left = js + c0 <= je ? (je - js - c0) / C + 1 : 0;  // partners not screened yet
   // i itself as a partner: position `self` in the item's list, if any
   int self = i - (js + c0);
@@ -1140,6 +1133,7 @@ __device__ __forceinline__ void pair_window_run(const PT *rec, int N, int i, int
       m0 = screen<NS, PT, PER>(rec, N, base + 32 * w * C, C, min(32, part - 32 * w), gi, k);
       if ((self >> 5) == w) m0 &= ~(1u << (self & 31));
       if (mb.words) *mask_word<NT>(mb, w) = m0;
+      some |= m0 != 0u;
     }
     // the next partner's record, or the molecule's own (which adds nothing)
     // where the current word is spent
@@ -1171,6 +1165,7 @@ __device__ __forceinline__ void pair_window_run(const PT *rec, int N, int i, int
     base += part * C;
     self -= part;
   }
+  return some;
 }
 
 // One work item's partner sums into `acc` (zero on entry).  FP32 pair math
@@ -1189,20 +1184,31 @@ __device__ __forceinline__ void pair_window(const PT *rec, int N, int i, int js,
     part.corr[0] = part.corr[1] = part.corr[2] = 0.0f;
     part.vir[0] = part.vir[1] = part.vir[2] = 0.0f;
     part.lj = part.clmb = 0.0f;
-    pair_window_run<NT, NS, QB, PT, PER, RECORDS>(rec, N, i, js, je, c0, C, compact, gi, ai, k, mb, part);
+    const bool some = pair_window_run<NT, NS, QB, PT, PER, RECORDS>(rec, N, i, js, je, c0, C, compact, gi, ai, k, mb, part);
 #pragma unroll
     for (int a = 0; a < NS; a++)
 #pragma unroll
-      for (int d = 0; d < 3; d++) acc.site[a][d] = (double)part.site[a][d];
+      for (int d = 0; d < 3; d++) acc.site[a][d] = some ? (double)part.site[a][d] : 0.0;
 #pragma unroll
     for (int d = 0; d < 3; d++) {
-      acc.corr[d] = (double)part.corr[d];
-      acc.vir[d] = (double)part.vir[d];
+      acc.corr[d] = some ? (double)part.corr[d] : 0.0;
+      acc.vir[d] = some ? (double)part.vir[d] : 0.0;
     }
-    acc.lj = (double)part.lj;
-    acc.clmb = (double)part.clmb;
+    acc.lj = some ? (double)part.lj : 0.0;
+    acc.clmb = some ? (double)part.clmb : 0.0;
   } else {
-    pair_window_run<NT, NS, QB, PT, PER, RECORDS>(rec, N, i, js, je, c0, C, compact, gi, ai, k, mb, acc);
+    const bool some = pair_window_run<NT, NS, QB, PT, PER, RECORDS>(rec, N, i, js, je, c0, C, compact, gi, ai, k, mb, acc);
+#pragma unroll
+    for (int a = 0; a < NS; a++)
+#pragma unroll
+      for (int d = 0; d < 3; d++) acc.site[a][d] = some ? acc.site[a][d] : 0.0;
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+      acc.corr[d] = some ? acc.corr[d] : 0.0;
+      acc.vir[d] = some ? acc.vir[d] : 0.0;
+    }
+    acc.lj = some ? acc.lj : 0.0;
+    acc.clmb = some ? acc.clmb : 0.0;
   }
 }
 

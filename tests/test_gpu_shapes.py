@@ -101,3 +101,22 @@ def test_global_path_parts_keep_the_bits(model, nmol, chunks, precision, abort, 
         for k in ("r", "v", "f", "q", "p", "n", "id", "scal"):
             assert np.array_equal(x[k], y[k]), k
     bt.close()
+
+
+@pytest.mark.parametrize("path", [2, 3])
+def test_replica_gone_non_finite_has_no_pairs(path):
+    """A replica whose positions are not numbers has no partner inside the
+    cutoff: forces, torques and energies are exactly zero, and the replica
+    beside it keeps its forces (1e-5 relative RMS, as above)."""
+    from helpers import oracle_for, rel_rms
+
+    s = _bulk(800, "TIP4P", nrep=2)
+    good = s.states[0].r
+    s.states[1].r = np.full_like(good, np.nan)
+    g = ra.REMDGPU(s, path=path)
+    bad = g.state(1)
+    assert np.all(bad["f"] == 0.0) and np.all(bad["n"] == 0.0)
+    assert np.all(g.averages(1)[:3] == 0.0)
+    o = oracle_for(s, 0)
+    o.initialize_property()
+    assert rel_rms(g.state(0)["f"], o.state()["f"]) < 1e-5
