@@ -65,8 +65,8 @@ struct JobParams {
                                 // global-state path, any 1..64 on the resident path)
   int precision;                // 0 mixed (FP32 pair, FP64 acc), 1 FP64
   int compact;                  // 1: screen partners by COM distance before the pair terms
-  int radix_min;                // resident path: molecules from which the neighbour sort is the
-                                // wave-ballot radix sort (the rank sort below; same order)
+  int bucket_min;               // resident path: molecules from which the neighbour sort goes by
+                                // buckets (by counting below; same order)
   int ens_fixed;                // resident path: 1 runs jobs of the ENS_*_NP ensembles on the
                                 // instantiations with the modes fixed (same bits as 0)
   double dt, dthalf;
@@ -105,9 +105,10 @@ struct ReplicaDesc {
 // Resident path: threads per workgroup (4 waves: one per SIMD of a CU).
 constexpr int RNT = 256;
 
-// Resident path: default molecule count from which the neighbour sort is
-// the radix sort rather than the rank sort.
-constexpr int RADIX_MIN_DEFAULT = 768;
+// Resident path: default molecule count from which the neighbour sort goes
+// by buckets rather than by counting (buckets are the faster at every size
+// measured, 144 to 1820; one wave counts up to 64 at once).
+constexpr int BUCKET_MIN_DEFAULT = 64;
 
 // Ensemble code of a job: tconstant 0..2, pconstant 0..3, confined 0..2, and
 // for tubes whether the partners are screened (ENS_SCREENED; bulk and slit

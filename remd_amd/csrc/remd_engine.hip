@@ -302,11 +302,10 @@ static void fill_params(const remd_gpu_desc *d, JobParams &J) {
   // are the windows of wide tubes: screen the partners first; narrow tubes'
   // windows are mostly inside it
   J.compact = d->confined == 1 ? tube_inside_fraction(d) < TUBE_SCREEN_BELOW : 1;
-  // the rank sort's O(N^2 / threads) comparisons lose to the radix sort's
-  // 16 passes from about this size (measured); REMD_SORT_RADIX_MIN overrides
+  // REMD_SORT_RADIX_MIN overrides the size from which the sort goes by buckets
   {
     const char *e = std::getenv("REMD_SORT_RADIX_MIN");
-    J.radix_min = e ? std::atoi(e) : RADIX_MIN_DEFAULT;
+    J.bucket_min = e ? std::atoi(e) : BUCKET_MIN_DEFAULT;
   }
   // REMD_ENSEMBLE_FIXED=0 runs every job on the instantiation that reads
   // the modes from the job (the tests compare the two)

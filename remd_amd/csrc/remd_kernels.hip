@@ -751,17 +751,18 @@ __device__ void radix_sort(uint64_t *keyA, uint16_t *idxA, uint64_t *keyB, uint1
 // Window bounds for nlane = 1 (src/molecules.cxx:556-583) on sorted keys z:
 // js = first index scanning down from i (cyclic) with z < z_i - w,
 // je = first index scanning up (cyclic) with z > z_i + w.
-__device__ inline int count_less(const double *z, int n, double x) {
-  int lo = 0, hi = n;  // first index with z >= x
-  while (lo < hi) {
+// `range(x, lo, hi)` bounds the searches: the answer for x lies in [lo, hi].
+template <typename Z>
+__device__ __forceinline__ int count_less(const Z *z, double x, int lo, int hi) {
+  while (lo < hi) {  // first index with z >= x
     const int mid = (lo + hi) >> 1;
     if (z[mid] < x) lo = mid + 1; else hi = mid;
   }
   return lo;
 }
-__device__ inline int count_leq(const double *z, int n, double x) {
-  int lo = 0, hi = n;  // first index with z > x
-  while (lo < hi) {
+template <typename Z>
+__device__ __forceinline__ int count_leq(const Z *z, double x, int lo, int hi) {
+  while (lo < hi) {  // first index with z > x
     const int mid = (lo + hi) >> 1;
     if (z[mid] <= x) lo = mid + 1; else hi = mid;
   }
@@ -769,30 +770,43 @@ __device__ inline int count_leq(const double *z, int n, double x) {
 }
 // The scan wraps at most twice for w < 2: a second wrap stops at once, on
 // index n - 1 (downward) or 0 (upward).
-__device__ inline void window_of(const double *z, int n, int i, double w, int &js, int &je) {
+template <typename Z, typename Range>
+__device__ __forceinline__ void window_of(const Z *z, int n, int i, double w, int &js, int &je, Range range) {
+  int lo, hi;
   double lb = z[i] - w;
-  int k = count_less(z, n, lb);
+  range(lb, lo, hi);
+  int k = count_less(z, lb, lo, hi);
   if (k >= 1) js = k - 1;
   else {
     lb += 1.0;
-    k = count_less(z, n, lb);
+    range(lb, lo, hi);
+    k = count_less(z, lb, lo, hi);
     js = (k >= 1) ? k - 1 : n - 1;
   }
   double ub = z[i] + w;
-  int m = count_leq(z, n, ub);
+  range(ub, lo, hi);
+  int m = count_leq(z, ub, lo, hi);
   if (m < n) je = m;
   else {
     ub -= 1.0;
-    m = count_leq(z, n, ub);
+    range(ub, lo, hi);
+    m = count_leq(z, ub, lo, hi);
     je = (m < n) ? m : 0;
   }
+}
+__device__ inline void window_of(const double *z, int n, int i, double w, int &js, int &je) {
+  window_of(z, n, i, w, js, je, [n](double, int &lo, int &hi) {
+    lo = 0;
+    hi = n;
+  });
 }
 
 // Contract (no reference counterpart): the window is the whole ring when
 // the scan wrapped onto i itself, or when the first key outside on one
 // side lies inside the other side's arc; the reference's js..je range then
 // misses pairs.  Same comparisons as the scan's bounds.
-__device__ inline bool window_full(const double *z, int i, double w, int js, int je) {
+template <typename Z>
+__device__ __forceinline__ bool window_full(const Z *z, int i, double w, int js, int je) {
   const bool a_up = (js > i) ? (z[js] <= z[i] + w) : (z[js] <= (z[i] + w) - 1.0);
   const bool b_dn = (je < i) ? (z[je] >= z[i] - w) : (z[je] >= (z[i] - w) + 1.0);
   return js == i || je == i || a_up || b_dn;
@@ -1941,85 +1955,202 @@ __device__ inline LdsR carve_resident(char *smem, int N, int prec, bool site_dbg
   return L;
 }
 
-// Sorted position rk[i] of each key ax[i] (stable: equal keys keep their
-// order) by the wave-ballot radix sort of the keys' order-preserving bit
-// patterns, in `region` (20 N bytes + the digit counts): keys A/B at 0 and
-// 8N, indices A/B at 16N and 18N, counts at 20N; 16 passes leave the result
-// in A.  rk (N 16-bit entries) must lie outside [0, 8N) and [16N, ...).
-// Out of line: inlined into the resident kernel it perturbs the register
-// allocation of the whole step loop.
-template <int NT>
-__device__ __attribute__((noinline)) void radix_ranks(const double *ax, int N, char *region, uint16_t *rk) {
-  uint64_t *keyA = (uint64_t *)region, *keyB = keyA + N;
-  uint16_t *idxA = (uint16_t *)(region + 16 * N), *idxB = idxA + N;
-  int *cnt = (int *)(region + 20 * N);
-  for (int i = threadIdx.x; i < N; i += NT) {
-    const uint64_t u = (uint64_t)__double_as_longlong(ax[i] + 0.0);  // -0.0 -> +0.0
-    keyA[i] = (u >> 63) ? ~u : (u | (1ull << 63));
-    idxA[i] = (uint16_t)i;
-  }
-  __syncthreads();
-  radix_sort<NT>(keyA, idxA, keyB, idxB, cnt, N);
-  for (int k = threadIdx.x; k < N; k += NT) rk[idxA[k]] = (uint16_t)k;
+// LDS seen as such in an out-of-line function (a generic pointer would make
+// every access there a flat one).
+#define REMD_LDS __attribute__((address_space(3)))
+
+// Bucket of a sort key among n: monotone in the order of the keys' bit
+// patterns (sign first), so a key in a lower bucket is smaller.
+__device__ __forceinline__ int bucket_of(double z, int n) {
+  const double t = z * (double)n;
+  if (t != t) return __double2hiint(z) < 0 ? 0 : n - 1;
+  return t >= (double)n ? n - 1 : (t >= 0.0 ? (int)t : 0);
 }
 
-// Stable rank sort of the sort-axis coordinate in LDS (the same order as a
-// stable sort on the double keys: rank = #smaller + #equal-and-earlier),
-// permutation of the state, then the windows by binary search on the sorted
-// keys (src/molecules.cxx:541-585 semantics; raw js/je and the whole-ring
-// flag go to win_dbg when given).
+// Region-0 layout of the bucket sort: keys (8 N), ranks (2 N), bucket heads
+// (N + 1 and a status word); the rest -- members (2 N) and their keys (8 N)
+// -- is scratch of bucket_ranks and staging afterwards.
+__host__ __device__ inline int bucket_heads(int nmol) { return align16(10 * nmol); }
+__host__ __device__ inline int bucket_scratch(int nmol) { return align16(bucket_heads(nmol) + 4 * nmol + 32); }
+__host__ __device__ inline int bucket_bytes(int nmol) { return bucket_scratch(nmol) + 8 * nmol + align16(2 * nmol); }
+
+// Sorted position of each of the N keys in region 0 (stable: equal keys keep
+// their order; the order of the keys' bit patterns, so a NaN has its place
+// too) as 16-bit ranks, the keys left sorted, and the bucket heads: head[b] =
+// keys in lower buckets.  N buckets of equal width over [0, 1): counted and
+// filled through LDS atomics in any order, then each key compares itself
+// with its own bucket's members, so the ranks do not depend on that order.
+// O(N) where the keys are spread (the molecules of a fluid), N^2 / NT
+// comparisons at worst.  The binary searches of the windows then start from
+// the bucket of their bound.  Kernel time of an interval against the 16-pass
+// wave-ballot radix sort and full searches: 1820 TIP4P 17.9 -> 16.5 ms, 1374
+// TIP5P 22.7 -> 21.8 ms; against count_ranks: 512 TIP5P 6.90 -> 6.65 ms, 256
+// TIP4P FP64 3.61 -> 3.57 ms, 144 TIP4P 1.312 -> 1.290 ms.
+// Returns whether a key was a NaN (the heads then bound no search).  Out of
+// line: inlined into the resident kernel it perturbs the register allocation
+// of the whole step loop.
+template <int NT>
+__device__ __attribute__((noinline)) bool bucket_ranks(REMD_LDS char *region, int N) {
+  REMD_LDS double *z = (REMD_LDS double *)region;
+  REMD_LDS uint16_t *rk = (REMD_LDS uint16_t *)(region + 8 * N);
+  REMD_LDS int *head = (REMD_LDS int *)(region + bucket_heads(N));
+  REMD_LDS int *status = head + N + 1;  // NaN seen, then a total per wave
+  REMD_LDS uint64_t *mkey = (REMD_LDS uint64_t *)(region + bucket_scratch(N));
+  REMD_LDS uint16_t *member = (REMD_LDS uint16_t *)(mkey + N);
+  const int lane = threadIdx.x & (WAVE - 1), wv = threadIdx.x / WAVE;
+  for (int b = threadIdx.x; b < N; b += NT) head[b] = 0;
+  if (threadIdx.x == 0) *status = 0;
+  __syncthreads();
+  for (int i = threadIdx.x; i < N; i += NT) {
+    const double x = z[i];
+    rk[i] = (uint16_t)__hip_atomic_fetch_add(&head[bucket_of(x, N)], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    if (x != x) *status = 1;
+  }
+  __syncthreads();
+  // counts -> heads: runs of q per thread, scanned over the wave, then over
+  // the waves
+  const int q = (N + NT - 1) / NT;
+  const int b0 = min(N, (int)threadIdx.x * q), b1 = min(N, b0 + q);
+  int own = 0;
+  for (int b = b0; b < b1; b++) own += head[b];
+  int sum = own;
+#pragma unroll
+  for (int d = 1; d < WAVE; d <<= 1) {
+    const int up = __shfl_up(sum, d, WAVE);
+    sum += lane >= d ? up : 0;
+  }
+  if (lane == WAVE - 1) status[1 + wv] = sum;
+  __syncthreads();
+  int at = sum - own;
+#pragma unroll
+  for (int w = 0; w < NT / WAVE; w++) at += w < wv ? status[1 + w] : 0;
+  for (int b = b0; b < b1; b++) {
+    const int c = head[b];
+    head[b] = at;
+    at += c;
+  }
+  if (threadIdx.x == 0) head[N] = N;
+  __syncthreads();
+  for (int i = threadIdx.x; i < N; i += NT) {
+    const double x = z[i];
+    const uint64_t u = (uint64_t)__double_as_longlong(x);
+    const int k = head[bucket_of(x, N)] + rk[i];
+    mkey[k] = (u >> 63) ? ~u : (u | (1ull << 63));
+    member[k] = (uint16_t)i;
+  }
+  __syncthreads();
+  for (int k = threadIdx.x; k < N; k += NT) {
+    const uint64_t key = mkey[k];
+    const int i = member[k];
+    const double x = __longlong_as_double((long long)((key >> 63) ? key & ~(1ull << 63) : ~key));
+    const int b = bucket_of(x, N), e = head[b + 1];
+    int r = head[b];
+    for (int m = r; m < e; m++) {
+      const uint64_t o = mkey[m];
+      r += (o < key || (o == key && member[m] < i)) ? 1 : 0;
+    }
+    rk[i] = (uint16_t)r;
+    z[r] = x;
+  }
+  __syncthreads();
+  return *status != 0;
+}
+
+// The same ranks by counting: rank = #smaller + #equal-and-earlier, the N x N
+// comparisons split into (molecule, segment of partners) items so that every
+// thread takes part: the segment count minimises the longest thread's
+// comparisons; the segments' counts meet in an integer per molecule
+// (order-free).
+template <int NT>
+__device__ __attribute__((noinline)) void count_ranks(REMD_LDS char *region, int N) {
+  REMD_LDS double *z = (REMD_LDS double *)region;
+  REMD_LDS uint16_t *rk = (REMD_LDS uint16_t *)(region + 8 * N);
+  REMD_LDS int *cnt = (REMD_LDS int *)(region + align16(10 * N));
+  int nseg = 1, best = 1 << 30;
+  for (int g = 1; g <= 8; g++) {
+    const int len = (N + g - 1) / g;
+    const int cost = ((N * g + NT - 1) / NT) * len + 8 * g;
+    if (cost < best) {
+      best = cost;
+      nseg = g;
+    }
+  }
+  const int len = (N + nseg - 1) / nseg;
+  for (int i = threadIdx.x; i < N; i += NT) cnt[i] = 0;
+  __syncthreads();
+  for (int t = threadIdx.x; t < N * nseg; t += NT) {
+    const int i = t % N, seg = t / N;
+    const double zi = z[i];
+    const int j0 = seg * len, j1 = min(N, j0 + len);
+    int r = 0;
+#pragma unroll 8
+    for (int j = j0; j < j1; ++j) {
+      const double zj = z[j];
+      r += (j < i) ? (zj <= zi ? 1 : 0) : (zj < zi ? 1 : 0);
+    }
+    if (nseg == 1) cnt[i] = r;
+    else __hip_atomic_fetch_add(&cnt[i], r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < N; i += NT) rk[i] = (uint16_t)cnt[i];
+  __syncthreads();
+}
+
+// Windows of the sorted keys in region 0 (raw js / je and the whole-ring flag
+// to win_dbg when given); with `bounded` each search starts from the bucket
+// of its bound.
+template <int NT>
+__device__ __attribute__((noinline)) void sorted_windows(REMD_LDS char *region, int N, double w, bool bounded,
+                                                         REMD_LDS uint16_t *js_out, REMD_LDS uint16_t *je_out,
+                                                         int *win_dbg) {
+  const REMD_LDS double *z = (const REMD_LDS double *)region;
+  const REMD_LDS int *head = (const REMD_LDS int *)(region + bucket_heads(N));
+  for (int i = threadIdx.x; i < N; i += NT) {
+    int js, je;
+    window_of(z, N, i, w, js, je, [&](double x, int &lo, int &hi) {
+      const bool in = bounded && x == x;
+      lo = 0;
+      hi = N;
+      if (in) {
+        const int b = bucket_of(x, N);
+        lo = head[b];
+        hi = head[b + 1];
+      }
+    });
+    const bool full = window_full(z, i, w, js, je);
+    if (win_dbg) {
+      win_dbg[3 * i] = js;
+      win_dbg[3 * i + 1] = je;
+      win_dbg[3 * i + 2] = full ? 1 : 0;
+    }
+    if (js >= je) je += N;
+    if (full || !((js <= i && i <= je) || (js <= i + N && i + N <= je))) {
+      js = i + 1;
+      je = i + N - 1;
+    }
+    js_out[i] = (uint16_t)js;
+    je_out[i] = (uint16_t)je;
+  }
+  __syncthreads();
+}
+
+// Stable sort of the sort-axis coordinate in LDS, permutation of the state,
+// then the windows by binary search on the sorted keys
+// (src/molecules.cxx:541-585 semantics).
 template <int NT, int NS, int EM = ENS_RUNTIME>
 __device__ void rank_sort_resident(JRef J, double *mol, int *mid, int N, double Laxis,
                                    double margin, const LdsR &S, int *win_dbg) {
   double *z = (double *)S.region0;
-  uint16_t *rk = (uint16_t *)(S.region0 + 8 * N);
-  double *ax = mol + (F_RX + sort_axis_of<EM>(J)) * N;
-  // large replicas: the wave-ballot radix sort of the keys' order-preserving
-  // bit patterns (stable, so the same order as the rank sort), in region 0:
-  // keys A/B at 0 and 8N bytes, indices A/B at 16N and 18N, digit counts
-  // after; 16 passes leave the result in A.  rk then goes to [8N, 10N).
-  const int ng = ((N + NT - 1) / NT) * (NT / WAVE);
-  const bool radix = N >= J.radix_min && 20 * N + 4 * 17 * ng <= resident_region0(N, NS, J.precision);
-  if (radix) {
-    radix_ranks<NT>(ax, N, S.region0, rk);
-  } else {
-    // rank = #smaller + #equal-and-earlier, the N x N comparisons split into
-    // (molecule, segment of partners) items so that every thread takes part:
-    // the segment count minimises the longest thread's comparisons; the
-    // segments' counts meet in an integer per molecule (order-free)
-    int *cnt = (int *)(S.region0 + align16(10 * N));
-    int nseg = 1, best = 1 << 30;
-    for (int g = 1; g <= 8; g++) {
-      const int len = (N + g - 1) / g;
-      const int cost = ((N * g + NT - 1) / NT) * len + 8 * g;
-      if (cost < best) {
-        best = cost;
-        nseg = g;
-      }
-    }
-    const int len = (N + nseg - 1) / nseg;
-    for (int i = threadIdx.x; i < N; i += NT) {
-      z[i] = ax[i] + 0.0;  // -0.0 -> +0.0
-      cnt[i] = 0;
-    }
-    __syncthreads();
-    for (int t = threadIdx.x; t < N * nseg; t += NT) {
-      const int i = t % N, seg = t / N;
-      const double zi = z[i];
-      const int j0 = seg * len, j1 = min(N, j0 + len);
-      int r = 0;
-#pragma unroll 8
-      for (int j = j0; j < j1; ++j) {
-        const double zj = z[j];
-        r += (j < i) ? (zj <= zi ? 1 : 0) : (zj < zi ? 1 : 0);
-      }
-      if (nseg == 1) cnt[i] = r;
-      else atomicAdd(&cnt[i], r);
-    }
-    __syncthreads();
-    for (int i = threadIdx.x; i < N; i += NT) rk[i] = (uint16_t)cnt[i];
-  }
+  const uint16_t *rk = (const uint16_t *)(S.region0 + 8 * N);
+  const double *ax = mol + (F_RX + sort_axis_of<EM>(J)) * N;
+  // by buckets from bucket_min molecules on, where region 0 has the room (any
+  // size but the few molecules at the bottom); both give the same order
+  const bool buckets = N >= J.bucket_min && bucket_bytes(N) <= resident_region0(N, NS, J.precision);
+  bool bounded = false;  // the heads bound the searches
+  for (int i = threadIdx.x; i < N; i += NT) z[i] = ax[i] + 0.0;  // -0.0 -> +0.0
   __syncthreads();
+  if (buckets) bounded = !bucket_ranks<NT>((REMD_LDS char *)S.region0, N);
+  else count_ranks<NT>((REMD_LDS char *)S.region0, N);
   // permute the state through the larger of the pair-partial area (idle
   // during the sort) and the rest of region 0, as many fields per round as
   // fit.  F and n are not permuted: the force pass that follows every sort
@@ -2027,8 +2158,9 @@ __device__ void rank_sort_resident(JRef J, double *mol, int *mid, int N, double 
   // the NPF permuted ones: r, v (k < 6), then q, p.
   constexpr int NPF = NFIELD - 7;
   const int cap_part = S.part_n / N;
-  const int cap_r0 = (resident_region0(N, NS, J.precision) - align16(10 * N)) / (8 * N);
-  double *tmp = cap_part >= cap_r0 ? S.part : (double *)(S.region0 + align16(10 * N));
+  const int used = buckets ? bucket_scratch(N) : align16(10 * N);
+  const int cap_r0 = (resident_region0(N, NS, J.precision) - used) / (8 * N);
+  double *tmp = cap_part >= cap_r0 ? S.part : (double *)(S.region0 + used);
   const int fit = cap_part >= cap_r0 ? cap_part : cap_r0;
   const int per = fit < 1 ? 1 : (fit > NPF ? NPF : fit);
   for (int f0 = 0; f0 < NPF; f0 += per) {
@@ -2054,25 +2186,12 @@ __device__ void rank_sort_resident(JRef J, double *mol, int *mid, int N, double 
     for (int i = threadIdx.x; i < N; i += NT) mid[i] = ti[i];
     __syncthreads();
   }
-  const double w = (J.rcut + margin) / Laxis;
-  for (int i = threadIdx.x; i < N; i += NT) {
-    int js, je;
-    window_of(ax, N, i, w, js, je);
-    const bool full = window_full(ax, i, w, js, je);
-    if (win_dbg) {
-      win_dbg[3 * i] = js;
-      win_dbg[3 * i + 1] = je;
-      win_dbg[3 * i + 2] = full ? 1 : 0;
-    }
-    if (js >= je) je += N;
-    if (full || !((js <= i && i <= je) || (js <= i + N && i + N <= je))) {
-      js = i + 1;
-      je = i + N - 1;
-    }
-    S.js[i] = (uint16_t)js;
-    S.je[i] = (uint16_t)je;
+  if (!buckets) {
+    for (int i = threadIdx.x; i < N; i += NT) z[i] = ax[i];
+    __syncthreads();
   }
-  __syncthreads();
+  sorted_windows<NT>((REMD_LDS char *)S.region0, N, (J.rcut + margin) / Laxis, bounded, (REMD_LDS uint16_t *)S.js,
+                     (REMD_LDS uint16_t *)S.je, win_dbg);
 }
 
 // Window of the last sort, from the debug copy (MODE_FORCE without a sort).

@@ -120,3 +120,42 @@ def test_replica_gone_non_finite_has_no_pairs(path):
     o = oracle_for(s, 0)
     o.initialize_property()
     assert rel_rms(g.state(0)["f"], o.state()["f"]) < 1e-5
+
+
+@pytest.mark.parametrize("nmol,path,keys", [
+    (4, 0, "spread"), (63, 0, "spread"), (257, 0, "spread"),
+    (515, 3, "spread"),
+    (300, 0, "equal"),     # one bucket holds every key
+    (300, 0, "layers"),    # equal keys in a few buckets, some zeros of either sign
+    (300, 0, "outside"),   # keys below 0 and above 1: the outer buckets
+    (300, 0, "nan"),       # a key without a place in the searches
+])
+def test_bucket_sort_order_and_windows(nmol, path, keys, monkeypatch):
+    """The bucket sort gives the stable order of the sort coordinate, and the
+    windows the counting sort gives (except where a NaN leaves that sort
+    without an order)."""
+    s = _bulk(nmol, "TIP4P", nrep=1)
+    rng = np.random.RandomState(nmol)
+    z = rng.permutation(s.states[0].r[:, 2] + 0.3 / nmol * rng.rand(nmol))
+    if keys == "equal":
+        z[:] = 0.37
+    elif keys == "layers":
+        z = rng.randint(0, 5, nmol) / 5.0
+        z[z == 0.0] = np.where(rng.rand(int((z == 0.0).sum())) < 0.5, -0.0, 0.0)
+    elif keys == "outside":
+        z = 3.0 * z - 1.0
+    elif keys == "nan":
+        z[7] = np.nan
+    s.states[0].r[:, 2] = z
+    got = []
+    for least in (1, 10 ** 6):
+        monkeypatch.setenv("REMD_SORT_RADIX_MIN", str(least))
+        g = ra.REMDGPU(s, path=path)
+        g.set_debug(True)
+        g.compute_forces(True)
+        got.append((g.state(0)["id"], g.window(0, with_full=True)))
+    assert np.array_equal(got[0][0], np.argsort(z, kind="stable"))
+    if keys != "nan":
+        assert np.array_equal(got[1][0], got[0][0])
+        for a, b in zip(got[0][1], got[1][1]):
+            assert np.array_equal(a, b)
