@@ -5,7 +5,7 @@
 //   D6 D5 D4 D3 D2 D1 D2 D3 (PsPv) D4 | force | D5 D6
 //   (src/integrator.cxx:646-706, the CPU canonical order), with
 //   - the z-sorted neighbour window rebuilt every sort_interval steps by a
-//     wave-ballot LSD radix sort in LDS (replaces src/sort.cu +
+//     bucket sort in LDS (a radix sort where LDS is short; replaces src/sort.cu +
 //     src/quicksort.cu; window semantics of src/molecules.cxx:541-585),
 //   - M2A into LDS site records (FP32 centred COM + FP32 site offsets,
 //     rotated in FP64; src/molecules.cxx:319-360, src/rotation.h:29-48),
@@ -812,12 +812,186 @@ __device__ __forceinline__ bool window_full(const Z *z, int i, double w, int js,
   return js == i || je == i || a_up || b_dn;
 }
 
+// LDS seen as such in an out-of-line function (a generic pointer would make
+// every access there a flat one).
+#define REMD_LDS __attribute__((address_space(3)))
+
+// Bucket of a sort key among n: monotone in the order of the keys' bit
+// patterns (sign first), so a key in a lower bucket is smaller.
+__device__ __forceinline__ int bucket_of(double z, int n) {
+  const double t = z * (double)n;
+  if (t != t) return __double2hiint(z) < 0 ? 0 : n - 1;
+  return t >= (double)n ? n - 1 : (t >= 0.0 ? (int)t : 0);
+}
+
+// Region-0 layout of the bucket sort: keys (8 N), ranks (2 N), bucket heads
+// (N + 1 and a status word); the rest -- members (2 N) and their keys (8 N)
+// -- is scratch of bucket_ranks and staging afterwards.
+__host__ __device__ inline int bucket_heads(int nmol) { return align16(10 * nmol); }
+__host__ __device__ inline int bucket_scratch(int nmol) { return align16(bucket_heads(nmol) + 4 * nmol + 32); }
+__host__ __device__ inline int bucket_bytes(int nmol) { return bucket_scratch(nmol) + 8 * nmol + align16(2 * nmol); }
+
+// Sorted position of each of the N keys in region 0 (stable: equal keys keep
+// their order; the order of the keys' bit patterns, so a NaN has its place
+// too) as 16-bit ranks, the keys left sorted, and the bucket heads: head[b] =
+// keys in lower buckets.  N buckets of equal width over [0, 1): counted and
+// filled through LDS atomics in any order, then each key compares itself
+// with its own bucket's members, so the ranks do not depend on that order.
+// O(N) where the keys are spread (the molecules of a fluid), N^2 / NT
+// comparisons at worst.  The binary searches of the windows then start from
+// the bucket of their bound.  Kernel time of an interval against the 16-pass
+// wave-ballot radix sort and full searches: 1820 TIP4P 17.9 -> 16.5 ms, 1374
+// TIP5P 22.7 -> 21.8 ms, 2048 TIP4P on the global-state path 18.7 -> 17.75 ms;
+// against count_ranks: 512 TIP5P 6.90 -> 6.65 ms, 256 TIP4P FP64 3.61 -> 3.57 ms, 144 TIP4P 1.312 -> 1.290 ms.
+// RAW orders the keys' bits as unsigned integers (keys below zero last), as
+// the radix sort of the global-state path does.
+// Returns whether a key was a NaN (RAW: or negative); the heads then bound no
+// search.  Out of line: inlined into the resident kernel it perturbs the
+// register allocation of the whole step loop.
+template <int NT, bool RAW>
+__device__ __attribute__((noinline)) bool bucket_ranks(REMD_LDS char *region, int N) {
+  auto bucket = [N](double x) { return RAW && __double2hiint(x) < 0 ? N - 1 : bucket_of(x, N); };
+  REMD_LDS double *z = (REMD_LDS double *)region;
+  REMD_LDS uint16_t *rk = (REMD_LDS uint16_t *)(region + 8 * N);
+  REMD_LDS int *head = (REMD_LDS int *)(region + bucket_heads(N));
+  REMD_LDS int *status = head + N + 1;  // NaN seen, then a total per wave
+  REMD_LDS uint64_t *mkey = (REMD_LDS uint64_t *)(region + bucket_scratch(N));
+  REMD_LDS uint16_t *member = (REMD_LDS uint16_t *)(mkey + N);
+  const int lane = threadIdx.x & (WAVE - 1), wv = threadIdx.x / WAVE;
+  for (int b = threadIdx.x; b < N; b += NT) head[b] = 0;
+  if (threadIdx.x == 0) *status = 0;
+  __syncthreads();
+  for (int i = threadIdx.x; i < N; i += NT) {
+    const double x = z[i];
+    rk[i] = (uint16_t)__hip_atomic_fetch_add(&head[bucket(x)], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    if (x != x || (RAW && __double2hiint(x) < 0)) *status = 1;
+  }
+  __syncthreads();
+  // counts -> heads: runs of q per thread, scanned over the wave, then over
+  // the waves
+  const int q = (N + NT - 1) / NT;
+  const int b0 = min(N, (int)threadIdx.x * q), b1 = min(N, b0 + q);
+  int own = 0;
+  for (int b = b0; b < b1; b++) own += head[b];
+  int sum = own;
+#pragma unroll
+  for (int d = 1; d < WAVE; d <<= 1) {
+    const int up = __shfl_up(sum, d, WAVE);
+    sum += lane >= d ? up : 0;
+  }
+  if (lane == WAVE - 1) status[1 + wv] = sum;
+  __syncthreads();
+  int at = sum - own;
+#pragma unroll
+  for (int w = 0; w < NT / WAVE; w++) at += w < wv ? status[1 + w] : 0;
+  for (int b = b0; b < b1; b++) {
+    const int c = head[b];
+    head[b] = at;
+    at += c;
+  }
+  if (threadIdx.x == 0) head[N] = N;
+  __syncthreads();
+  for (int i = threadIdx.x; i < N; i += NT) {
+    const double x = z[i];
+    const uint64_t u = (uint64_t)__double_as_longlong(x);
+    const int k = head[bucket(x)] + rk[i];
+    mkey[k] = RAW ? u : (u >> 63) ? ~u : (u | (1ull << 63));
+    member[k] = (uint16_t)i;
+  }
+  __syncthreads();
+  for (int k = threadIdx.x; k < N; k += NT) {
+    const uint64_t key = mkey[k];
+    const int i = member[k];
+    const double x = __longlong_as_double((long long)(RAW ? key : (key >> 63) ? key & ~(1ull << 63) : ~key));
+    const int b = bucket(x), e = head[b + 1];
+    int r = head[b];
+    for (int m = r; m < e; m++) {
+      const uint64_t o = mkey[m];
+      r += (o < key || (o == key && member[m] < i)) ? 1 : 0;
+    }
+    rk[i] = (uint16_t)r;
+    z[r] = x;
+  }
+  __syncthreads();
+  return *status != 0;
+}
+
+// Windows of the sorted keys in region 0 (raw js / je and the whole-ring flag
+// to win_dbg when given); with `bounded` each search starts from the bucket
+// of its bound.
+template <int NT>
+__device__ __attribute__((noinline)) void sorted_windows(REMD_LDS char *region, int N, double w, bool bounded,
+                                                         REMD_LDS uint16_t *js_out, REMD_LDS uint16_t *je_out,
+                                                         int *win_dbg) {
+  const REMD_LDS double *z = (const REMD_LDS double *)region;
+  const REMD_LDS int *head = (const REMD_LDS int *)(region + bucket_heads(N));
+  for (int i = threadIdx.x; i < N; i += NT) {
+    int js, je;
+    window_of(z, N, i, w, js, je, [&](double x, int &lo, int &hi) {
+      const bool in = bounded && x == x;
+      lo = 0;
+      hi = N;
+      if (in) {
+        const int b = bucket_of(x, N);
+        lo = head[b];
+        hi = head[b + 1];
+      }
+    });
+    const bool full = window_full(z, i, w, js, je);
+    if (win_dbg) {
+      win_dbg[3 * i] = js;
+      win_dbg[3 * i + 1] = je;
+      win_dbg[3 * i + 2] = full ? 1 : 0;
+    }
+    if (js >= je) je += N;
+    if (full || !((js <= i && i <= je) || (js <= i + N && i + N <= je))) {
+      js = i + 1;
+      je = i + N - 1;
+    }
+    js_out[i] = (uint16_t)js;
+    je_out[i] = (uint16_t)je;
+  }
+  __syncthreads();
+}
+
 // Sort the replica's molecules by the sort-axis coordinate, permute every
 // state array, rebuild js/je (CalcForcePot's doSort branch,
 // src/molecules.cxx:543-585).
 template <int NT>
 __device__ void sort_and_window(JRef J, double *mol, int *mid, int N, double Laxis,
                                 double margin, const Lds &S, int *win_dbg) {
+  const int room = (int)((char *)S.js - S.region0);
+  if (bucket_bytes(N) <= room) {
+    // where region 0 holds the site records; else (records in global memory)
+    // the radix sort below makes do with 20 N bytes
+    double *z = (double *)S.region0;
+    const uint16_t *rk = (const uint16_t *)(S.region0 + 8 * N);
+    const double *col = mol + (F_RX + J.sort_axis) * N;
+    for (int i = threadIdx.x; i < N; i += NT) z[i] = col[i] + 0.0;  // -0.0 -> +0.0
+    __syncthreads();
+    const bool bounded = !bucket_ranks<NT, true>((REMD_LDS char *)S.region0, N);
+    // as many state arrays per round as fit
+    double *tmp = (double *)(S.region0 + bucket_scratch(N));
+    const int per = (room - bucket_scratch(N)) / (8 * N);
+    for (int f0 = 0; f0 < NFIELD; f0 += per) {
+      const int nf = min(per, NFIELD - f0);
+      double *block = mol + f0 * N;
+      for (int i = threadIdx.x; i < N; i += NT) {
+        const int ri = rk[i];
+        for (int f = 0; f < nf; ++f) tmp[f * N + ri] = block[f * N + i];
+      }
+      __syncthreads();
+      for (int k = threadIdx.x; k < nf * N; k += NT) block[k] = tmp[k];
+      __syncthreads();
+    }
+    int *ti = (int *)tmp;
+    for (int i = threadIdx.x; i < N; i += NT) ti[rk[i]] = mid[i];
+    __syncthreads();
+    for (int i = threadIdx.x; i < N; i += NT) mid[i] = ti[i];
+    sorted_windows<NT>((REMD_LDS char *)S.region0, N, (J.rcut + margin) / Laxis, bounded, (REMD_LDS uint16_t *)S.js,
+                       (REMD_LDS uint16_t *)S.je, win_dbg);
+    return;
+  }
   uint64_t *keyA = (uint64_t *)S.region0;
   uint64_t *keyB = keyA + N;
   uint16_t *idxA = (uint16_t *)(keyB + N);
@@ -1956,107 +2130,6 @@ __device__ inline LdsR carve_resident(char *smem, int N, int prec, bool site_dbg
   return L;
 }
 
-// LDS seen as such in an out-of-line function (a generic pointer would make
-// every access there a flat one).
-#define REMD_LDS __attribute__((address_space(3)))
-
-// Bucket of a sort key among n: monotone in the order of the keys' bit
-// patterns (sign first), so a key in a lower bucket is smaller.
-__device__ __forceinline__ int bucket_of(double z, int n) {
-  const double t = z * (double)n;
-  if (t != t) return __double2hiint(z) < 0 ? 0 : n - 1;
-  return t >= (double)n ? n - 1 : (t >= 0.0 ? (int)t : 0);
-}
-
-// Region-0 layout of the bucket sort: keys (8 N), ranks (2 N), bucket heads
-// (N + 1 and a status word); the rest -- members (2 N) and their keys (8 N)
-// -- is scratch of bucket_ranks and staging afterwards.
-__host__ __device__ inline int bucket_heads(int nmol) { return align16(10 * nmol); }
-__host__ __device__ inline int bucket_scratch(int nmol) { return align16(bucket_heads(nmol) + 4 * nmol + 32); }
-__host__ __device__ inline int bucket_bytes(int nmol) { return bucket_scratch(nmol) + 8 * nmol + align16(2 * nmol); }
-
-// Sorted position of each of the N keys in region 0 (stable: equal keys keep
-// their order; the order of the keys' bit patterns, so a NaN has its place
-// too) as 16-bit ranks, the keys left sorted, and the bucket heads: head[b] =
-// keys in lower buckets.  N buckets of equal width over [0, 1): counted and
-// filled through LDS atomics in any order, then each key compares itself
-// with its own bucket's members, so the ranks do not depend on that order.
-// O(N) where the keys are spread (the molecules of a fluid), N^2 / NT
-// comparisons at worst.  The binary searches of the windows then start from
-// the bucket of their bound.  Kernel time of an interval against the 16-pass
-// wave-ballot radix sort and full searches: 1820 TIP4P 17.9 -> 16.5 ms, 1374
-// TIP5P 22.7 -> 21.8 ms; against count_ranks: 512 TIP5P 6.90 -> 6.65 ms, 256
-// TIP4P FP64 3.61 -> 3.57 ms, 144 TIP4P 1.312 -> 1.290 ms.
-// Returns whether a key was a NaN (the heads then bound no search).  Out of
-// line: inlined into the resident kernel it perturbs the register allocation
-// of the whole step loop.
-template <int NT>
-__device__ __attribute__((noinline)) bool bucket_ranks(REMD_LDS char *region, int N) {
-  REMD_LDS double *z = (REMD_LDS double *)region;
-  REMD_LDS uint16_t *rk = (REMD_LDS uint16_t *)(region + 8 * N);
-  REMD_LDS int *head = (REMD_LDS int *)(region + bucket_heads(N));
-  REMD_LDS int *status = head + N + 1;  // NaN seen, then a total per wave
-  REMD_LDS uint64_t *mkey = (REMD_LDS uint64_t *)(region + bucket_scratch(N));
-  REMD_LDS uint16_t *member = (REMD_LDS uint16_t *)(mkey + N);
-  const int lane = threadIdx.x & (WAVE - 1), wv = threadIdx.x / WAVE;
-  for (int b = threadIdx.x; b < N; b += NT) head[b] = 0;
-  if (threadIdx.x == 0) *status = 0;
-  __syncthreads();
-  for (int i = threadIdx.x; i < N; i += NT) {
-    const double x = z[i];
-    rk[i] = (uint16_t)__hip_atomic_fetch_add(&head[bucket_of(x, N)], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    if (x != x) *status = 1;
-  }
-  __syncthreads();
-  // counts -> heads: runs of q per thread, scanned over the wave, then over
-  // the waves
-  const int q = (N + NT - 1) / NT;
-  const int b0 = min(N, (int)threadIdx.x * q), b1 = min(N, b0 + q);
-  int own = 0;
-  for (int b = b0; b < b1; b++) own += head[b];
-  int sum = own;
-#pragma unroll
-  for (int d = 1; d < WAVE; d <<= 1) {
-    const int up = __shfl_up(sum, d, WAVE);
-    sum += lane >= d ? up : 0;
-  }
-  if (lane == WAVE - 1) status[1 + wv] = sum;
-  __syncthreads();
-  int at = sum - own;
-#pragma unroll
-  for (int w = 0; w < NT / WAVE; w++) at += w < wv ? status[1 + w] : 0;
-  for (int b = b0; b < b1; b++) {
-    const int c = head[b];
-    head[b] = at;
-    at += c;
-  }
-  if (threadIdx.x == 0) head[N] = N;
-  __syncthreads();
-  for (int i = threadIdx.x; i < N; i += NT) {
-    const double x = z[i];
-    const uint64_t u = (uint64_t)__double_as_longlong(x);
-    const int k = head[bucket_of(x, N)] + rk[i];
-    mkey[k] = (u >> 63) ? ~u : (u | (1ull << 63));
-    member[k] = (uint16_t)i;
-  }
-  __syncthreads();
-  for (int k = threadIdx.x; k < N; k += NT) {
-    const uint64_t key = mkey[k];
-    const int i = member[k];
-    const double x = __longlong_as_double((long long)((key >> 63) ? key & ~(1ull << 63) : ~key));
-    const int b = bucket_of(x, N), e = head[b + 1];
-    int r = head[b];
-    for (int m = r; m < e; m++) {
-      const uint64_t o = mkey[m];
-      r += (o < key || (o == key && member[m] < i)) ? 1 : 0;
-    }
-    rk[i] = (uint16_t)r;
-    z[r] = x;
-  }
-  __syncthreads();
-  return *status != 0;
-}
-
 // The same ranks by counting: rank = #smaller + #equal-and-earlier, the N x N
 // comparisons split into (molecule, segment of partners) items so that every
 // thread takes part: the segment count minimises the longest thread's
@@ -2097,44 +2170,6 @@ __device__ __attribute__((noinline)) void count_ranks(REMD_LDS char *region, int
   __syncthreads();
 }
 
-// Windows of the sorted keys in region 0 (raw js / je and the whole-ring flag
-// to win_dbg when given); with `bounded` each search starts from the bucket
-// of its bound.
-template <int NT>
-__device__ __attribute__((noinline)) void sorted_windows(REMD_LDS char *region, int N, double w, bool bounded,
-                                                         REMD_LDS uint16_t *js_out, REMD_LDS uint16_t *je_out,
-                                                         int *win_dbg) {
-  const REMD_LDS double *z = (const REMD_LDS double *)region;
-  const REMD_LDS int *head = (const REMD_LDS int *)(region + bucket_heads(N));
-  for (int i = threadIdx.x; i < N; i += NT) {
-    int js, je;
-    window_of(z, N, i, w, js, je, [&](double x, int &lo, int &hi) {
-      const bool in = bounded && x == x;
-      lo = 0;
-      hi = N;
-      if (in) {
-        const int b = bucket_of(x, N);
-        lo = head[b];
-        hi = head[b + 1];
-      }
-    });
-    const bool full = window_full(z, i, w, js, je);
-    if (win_dbg) {
-      win_dbg[3 * i] = js;
-      win_dbg[3 * i + 1] = je;
-      win_dbg[3 * i + 2] = full ? 1 : 0;
-    }
-    if (js >= je) je += N;
-    if (full || !((js <= i && i <= je) || (js <= i + N && i + N <= je))) {
-      js = i + 1;
-      je = i + N - 1;
-    }
-    js_out[i] = (uint16_t)js;
-    je_out[i] = (uint16_t)je;
-  }
-  __syncthreads();
-}
-
 // Stable sort of the sort-axis coordinate in LDS, permutation of the state,
 // then the windows by binary search on the sorted keys
 // (src/molecules.cxx:541-585 semantics).
@@ -2150,7 +2185,7 @@ __device__ void rank_sort_resident(JRef J, double *mol, int *mid, int N, double 
   bool bounded = false;  // the heads bound the searches
   for (int i = threadIdx.x; i < N; i += NT) z[i] = ax[i] + 0.0;  // -0.0 -> +0.0
   __syncthreads();
-  if (buckets) bounded = !bucket_ranks<NT>((REMD_LDS char *)S.region0, N);
+  if (buckets) bounded = !bucket_ranks<NT, false>((REMD_LDS char *)S.region0, N);
   else count_ranks<NT>((REMD_LDS char *)S.region0, N);
   // permute the state through the larger of the pair-partial area (idle
   // during the sort) and the rest of region 0, as many fields per round as

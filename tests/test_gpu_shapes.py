@@ -159,3 +159,33 @@ def test_bucket_sort_order_and_windows(nmol, path, keys, monkeypatch):
         assert np.array_equal(got[1][0], got[0][0])
         for a, b in zip(got[0][1], got[1][1]):
             assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("nmol,precision,keys", [
+    (65, 0, "spread"), (515, 0, "spread"), (700, 1, "spread"),
+    (300, 0, "outside"),    # keys below zero come last in this path's order
+    (300, 0, "nan"),
+    (1100, 1, "spread"),    # records in global memory: the radix sort
+])
+def test_global_path_sort_order_and_windows(nmol, precision, keys):
+    """The global-state path's order is that of the keys' bits as unsigned
+    integers, stable; its windows those of the split-global path."""
+    s = _bulk(nmol, "TIP4P", nrep=1)
+    rng = np.random.RandomState(nmol)
+    z = rng.permutation(s.states[0].r[:, 2] + 0.3 / nmol * rng.rand(nmol))
+    if keys == "outside":
+        z = 3.0 * z - 1.0
+    elif keys == "nan":
+        z[7] = np.nan
+    s.states[0].r[:, 2] = z
+    got = []
+    for path, prec in ((ra.PATH_GLOBAL, precision), (ra.PATH_SPLIT, 0)):
+        g = ra.REMDGPU(s, precision=prec, path=path)
+        g.set_debug(True)
+        g.compute_forces(True)
+        got.append((g.state(0)["id"], g.window(0, with_full=True)))
+    assert np.array_equal(got[0][0], np.argsort((z + 0.0).view(np.uint64), kind="stable"))
+    if keys == "spread":
+        assert np.array_equal(got[1][0], got[0][0])
+        for a, b in zip(got[0][1], got[1][1]):
+            assert np.array_equal(a, b)
