@@ -362,7 +362,8 @@ static void fill_params(const remd_gpu_desc *d, JobParams &J) {
 // device of ncu CUs: all of them resident at once, one per CU, the parts of
 // a replica on one XCD (block indices equal mod 8), and enough molecules for
 // a whole wave of work items per part.  100 steps of 8 replicas of 2048
-// TIP4P: 71.0 ms on 8 workgroups, 18.6 ms on 64.  Below GLOBAL_SPLIT_MIN
+// TIP4P: 71.0 ms on 8 workgroups, 18.6 ms on 64 (17.7 ms now, with the bucket
+// sort).  Below GLOBAL_SPLIT_MIN
 // (jobs that ask for this path) one workgroup per replica as before.
 constexpr int GLOBAL_SPLIT_MIN = 512;
 static int global_parts_max(int ncu, int nrep, int nmol, int chunks) {
