@@ -842,7 +842,10 @@ __host__ __device__ inline int bucket_bytes(int nmol) { return bucket_scratch(nm
 // the bucket of their bound.  Kernel time of an interval against the 16-pass
 // wave-ballot radix sort and full searches: 1820 TIP4P 17.9 -> 16.5 ms, 1374
 // TIP5P 22.7 -> 21.8 ms, 2048 TIP4P on the global-state path 18.7 -> 17.75 ms;
-// against count_ranks: 512 TIP5P 6.90 -> 6.65 ms, 256 TIP4P FP64 3.61 -> 3.57 ms, 144 TIP4P 1.312 -> 1.290 ms.
+// against count_ranks: 512 TIP5P 6.90 -> 6.65 ms, 256 TIP4P FP64 3.61 -> 3.57
+// ms, 144 TIP4P 1.312 -> 1.290 ms.  With a replica gone non-finite, one bucket
+// of 1820 keys: 33.5 ms; four members loaded ahead made that 22.5, but every
+// ordinary sort longer (144 TIP4P 1.280 -> 1.296 ms, 1374 TIP5P 21.45 -> 21.7).
 // RAW orders the keys' bits as unsigned integers (keys below zero last), as
 // the radix sort of the global-state path does.
 // Returns whether a key was a NaN (RAW: or negative); the heads then bound no
